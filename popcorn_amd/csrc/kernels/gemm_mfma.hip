@@ -6,16 +6,13 @@
 // With the MFMA lane layout of mfma.hpp both operands are 16-byte runs
 // along K of a row of A or of Bt.
 //
-// A block computes a BM x BN tile (128 or 256 each; 4 or 8 waves, each wave
-// a 64 x 64 or 128 x 64 piece of 32 x 32 MFMA tiles; the host picks the tile
-// shape per GEMM so the tile count fills the 256 CUs evenly). K advances 64
-// at a time through two LDS stages
-// (rows padded to 72 elements, so the 32 rows a fragment load touches fall
-// in distinct banks); the next stage's global loads are in registers while
-// the current stage is multiplied. Tiles are assigned XCD by XCD (blocks
-// are dealt round-robin to the 8 XCDs, so block b runs on XCD b % 8) and,
-// within an XCD's range, in groups of 8 tile rows, so the A and B panels a
-// group shares stay in that XCD's L2.
+// A block computes a BM x BN tile (64 to 256 by 64 to 384) on 4, 8 or 12
+// waves of 32 x 32 MFMA tiles; the host picks the tile, and for small grids
+// a split of K over several blocks, so the blocks fill the 256 CUs. The
+// operands go global -> LDS directly, several stages in flight. Tiles are
+// assigned XCD by XCD (blocks are dealt round-robin to the 8 XCDs, so block b
+// runs on XCD b % 8) and, within an XCD's range, in groups of 8 tile rows, so
+// the A and B panels a group shares stay in that XCD's L2.
 #include <type_traits>
 
 #include "mfma.hpp"
@@ -26,18 +23,19 @@ using pk::f32x16;
 using pk::Mma;
 using pk::u32x4;
 
-constexpr int BK = 64;
-constexpr int LDK = BK + 8;  // padded LDS row, in elements
 constexpr int kXcds = 8;
 constexpr int kGroupM = 8;
 
 __device__ inline void group_tile(uint32_t pid, uint32_t nM, uint32_t nN, uint32_t &pm, uint32_t &pn);
+// Unit of block b of `units`: block b runs on XCD b % 8, and each XCD takes a
+// contiguous range of the units (the first units % 8 XCDs one more each).
+__device__ inline uint32_t xcd_unit(uint32_t b, uint32_t units) {
+    const uint32_t x = b % kXcds, per = units / kXcds, more = units % kXcds;
+    return x * per + min(x, more) + b / kXcds;
+}
 // Tile (pm, pn) of block b: XCD-contiguous ranges, grouped rows within.
 __device__ inline void tile_of(uint32_t b, uint32_t nM, uint32_t nN, uint32_t &pm, uint32_t &pn) {
-    const uint32_t total = nM * nN;
-    uint32_t pid = b;
-    if (total % kXcds == 0) pid = (b % kXcds) * (total / kXcds) + b / kXcds;
-    group_tile(pid, nM, nN, pm, pn);
+    group_tile(xcd_unit(b, nM * nN), nM, nN, pm, pn);
 }
 // Split-K grids (tiles x splits): the XCD-contiguous ranges run over the
 // (split, tile) units, so an XCD's blocks share one split's K range and a
@@ -45,9 +43,8 @@ __device__ inline void tile_of(uint32_t b, uint32_t nM, uint32_t nN, uint32_t &p
 // down: 327 -> 314 us against ranges over the tiles alone, where every
 // XCD read all of A).
 __device__ inline void split_tile_of(uint32_t nM, uint32_t nN, uint32_t &pm, uint32_t &pn, uint32_t &split) {
-    const uint32_t tiles = nM * nN, units = tiles * gridDim.y;
-    const uint32_t b = blockIdx.x + blockIdx.y * gridDim.x;
-    const uint32_t u = units % kXcds == 0 ? (b % kXcds) * (units / kXcds) + b / kXcds : b;
+    const uint32_t tiles = nM * nN;
+    const uint32_t u = xcd_unit(blockIdx.x + blockIdx.y * gridDim.x, tiles * gridDim.y);
     split = u / tiles;
     group_tile(u % tiles, nM, nN, pm, pn);
 }
@@ -61,127 +58,12 @@ __device__ inline void group_tile(uint32_t pid, uint32_t nM, uint32_t nN, uint32
     pn = (pid % inGroup) / gm;
 }
 
-// BM x BN block tile on WM_N x WN_N waves; each wave a (BM / WM_N) x
-// (BN / WN_N) tile of 32 x 32 MFMA tiles.
-template <typename T, typename O, int BM, int BN, int WM_N, int WN_N>
-__device__ void gemm_nt(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                        typename O::storage *__restrict__ C, const MatmulConstants &p) {
-    constexpr int kThreads = 64 * WM_N * WN_N;
-    constexpr int WM = BM / WM_N, WN = BN / WN_N;
-    constexpr int TM = WM / 32, TN = WN / 32;
-    constexpr int kChunksA = BM * BK / 8 / kThreads, kChunksB = BN * BK / 8 / kThreads;
-    static_assert(kChunksA * kThreads * 8 == BM * BK && kChunksB * kThreads * 8 == BN * BK, "tile / thread count");
-    // Two stages of [A rows | B rows], each row LDK elements. The array is
-    // declared here (not passed in) so every access stays an LDS access.
-    constexpr int kStage = (BM + BN) * LDK;
-    __shared__ __attribute__((aligned(16))) uint16_t smem[2 * kStage];
-    auto sA = [&](int buf) { return smem + buf * kStage; };
-    auto sB = [&](int buf) { return smem + buf * kStage + BM * LDK; };
-
-    const uint32_t M = p.M, N = p.N, K = p.K;
-    const uint32_t nM = (M + BM - 1) / BM, nN = (N + BN - 1) / BN;
-    uint32_t pm, pn;
-    tile_of(blockIdx.x, nM, nN, pm, pn);
-    const uint32_t bm = pm * BM, bn = pn * BN;
-    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const uint32_t wm = (wave / WN_N) * WM, wn = (wave % WN_N) * WN;
-
-    // Global chunk c of a stage: row c / 8 of the tile, elements (c % 8) * 8 .. +8
-    // of the stage's K range. Rows past M (N) and K past the end read a valid
-    // address and are zeroed when stored to LDS (the mask is applied there,
-    // after the stage's multiply, so the loads stay in flight meanwhile).
-    u32x4 ra[kChunksA], rb[kChunksB];
-    uint32_t okA = 0, okB = 0;
-    auto gload = [&](uint32_t k0) {
-        okA = okB = 0;
-#pragma unroll
-        for (int i = 0; i < kChunksA; ++i) {
-            const uint32_t c = t + i * kThreads, r = c >> 3, k = k0 + (c & 7) * 8;
-            const uint32_t ar = bm + r;
-            const bool kin = k < K;
-            ra[i] = *reinterpret_cast<const u32x4 *>(A + (uint64_t)min(ar, M - 1) * K + (kin ? k : 0u));
-            okA |= (ar < M && kin) ? 1u << i : 0u;
-        }
-#pragma unroll
-        for (int i = 0; i < kChunksB; ++i) {
-            const uint32_t c = t + i * kThreads, r = c >> 3, k = k0 + (c & 7) * 8;
-            const uint32_t br = bn + r;
-            const bool kin = k < K;
-            rb[i] = *reinterpret_cast<const u32x4 *>(B + (uint64_t)min(br, N - 1) * K + (kin ? k : 0u));
-            okB |= (br < N && kin) ? 1u << i : 0u;
-        }
-    };
-    auto lstore = [&](int buf) {
-        const u32x4 zero = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int i = 0; i < kChunksA; ++i) {
-            const uint32_t c = t + i * kThreads, r = c >> 3, kc = (c & 7) * 8;
-            *reinterpret_cast<u32x4 *>(&sA(buf)[r * LDK + kc]) = (okA >> i) & 1u ? ra[i] : zero;
-        }
-#pragma unroll
-        for (int i = 0; i < kChunksB; ++i) {
-            const uint32_t c = t + i * kThreads, r = c >> 3, kc = (c & 7) * 8;
-            *reinterpret_cast<u32x4 *>(&sB(buf)[r * LDK + kc]) = (okB >> i) & 1u ? rb[i] : zero;
-        }
-    };
-
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for (int mi = 0; mi < TM; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < TN; ++ni)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[mi][ni][i] = 0.0f;
-
-    auto compute = [&](int buf) {
-#pragma unroll
-        for (int kk = 0; kk < BK / 16; ++kk) {
-            const uint32_t ko = kk * 16 + (lane >> 5) * 8;
-            u32x4 fa[TM], fb[TN];
-#pragma unroll
-            for (int mi = 0; mi < TM; ++mi)
-                fa[mi] = *reinterpret_cast<const u32x4 *>(&sA(buf)[(wm + mi * 32 + (lane & 31)) * LDK + ko]);
-#pragma unroll
-            for (int ni = 0; ni < TN; ++ni)
-                fb[ni] = *reinterpret_cast<const u32x4 *>(&sB(buf)[(wn + ni * 32 + (lane & 31)) * LDK + ko]);
-#pragma unroll
-            for (int mi = 0; mi < TM; ++mi)
-#pragma unroll
-                for (int ni = 0; ni < TN; ++ni) acc[mi][ni] = Mma<T>::run(fa[mi], fb[ni], acc[mi][ni]);
-        }
-    };
-
-    const uint32_t nk = (K + BK - 1) / BK;
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    for (uint32_t kt = 0; kt < nk; ++kt) {
-        const int cur = kt & 1;
-        if (kt + 1 < nk) gload((kt + 1) * BK);
-        compute(cur);
-        if (kt + 1 < nk) lstore(cur ^ 1);
-        __syncthreads();
-    }
-
-#pragma unroll
-    for (int mi = 0; mi < TM; ++mi) {
-#pragma unroll
-        for (int ni = 0; ni < TN; ++ni) {
-            const uint32_t col = bn + wn + ni * 32 + (lane & 31);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const uint32_t row = bm + wm + mi * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-                if (row < M && col < N) C[(uint64_t)row * N + col] = O::store(acc[mi][ni][i]);
-            }
-        }
-    }
-}
-
 // ---- direct-to-LDS pipeline ----------------------------------------------------
-// The same tile product with the operand tiles copied global -> LDS by
-// global_load_lds_dwordx4 (lane l of a wave instruction writes 16 bytes at
-// M0 + 16 l, checked on gfx950), kStagesD stages of BKD = 32 in flight and
-// no staging registers. A stage holds BM + BN rows of 64 bytes (4 chunks);
+// BM x BN block tile on WM_N x WN_N waves; each wave a (BM / WM_N) x
+// (BN / WN_N) tile of 32 x 32 MFMA tiles. The operand tiles are copied
+// global -> LDS by global_load_lds_dwordx4 (lane l of a wave instruction
+// writes 16 bytes at M0 + 16 l, checked on gfx950), kStagesD stages of
+// BKD = 32 in flight and no staging registers. A stage holds BM + BN rows of 64 bytes (4 chunks);
 // chunk kc of row r sits in slot kc ^ ((r >> 2) & 3), so the 16 rows a
 // fragment read touches (lanes 16 at a time) fall in 16 distinct 4-bank
 // groups. Needs K % 32 == 0 (a chunk past K cannot be zero-filled here).
@@ -366,18 +248,21 @@ __device__ void gemm_nt_direct(const uint16_t *__restrict__ A, const uint16_t *_
     }
 }
 
-// ---- whole-line pipeline ("e" tiles, K % 64 == 0) ---------------------------
+// ---- whole-line pipeline ("e" and "f" tiles) ---------------------------------
 // The same tile product with K = 64 per stage: 128-byte LDS rows, so each
 // copy instruction (8 lanes per row, buffer_load ... lds) requests whole
 // 128-byte lines. The 64-byte rows of the pipeline above fetch each line
 // twice, a stage apart, and the L2 -> LDS copy rate bounds those tiles
 // (config-5 gate 283 -> 261 us, down 322 -> 290 us, bit for bit the same
-// products). Two stage buffers; the copies of stage kt + 2 are issued at
-// the barrier before the last K-16 quarter of stage kt. Chunk c of row r
-// sits in slot c ^ ((r >> 1) & 7): the 16 rows a quarter-wave of a
-// fragment read touches cover all 64 banks.
+// products). NS stage buffers; the copies of stage kt + NS are issued at
+// the barrier before the last K-16 quarter of stage kt. Two ("e") leave LDS
+// for large tiles or two blocks per CU. A grid of one small tile per CU is
+// bound by the copies' latency instead: four ("f") took M 250, K 2304, N 4096
+// from 25.2 us (128 x 128, two stages) to 13.3 on 64 x 64 tiles (three
+// stages: 14.9). Chunk c of row r sits in slot c ^ ((r >> 1) & 7): the 16
+// rows a quarter-wave of a fragment read touches cover all 64 banks.
 constexpr int BK64 = 64;
-template <typename T, typename O, int BM, int BN, int WM_N, int WN_N, bool SPLITK = false>
+template <typename T, typename O, int BM, int BN, int WM_N, int WN_N, bool SPLITK = false, int NS = 2>
 __device__ void gemm_nt_lines(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                  typename O::storage *__restrict__ C, const MatmulConstants &p,
                                  float *__restrict__ P = nullptr) {
@@ -391,7 +276,8 @@ __device__ void gemm_nt_lines(const uint16_t *__restrict__ A, const uint16_t *__
     constexpr int kInst = (BM + BN) / 8, kInstA = BM / 8;
     constexpr int kPer = (kInst + NW - 1) / NW;  // per wave, rounded up
     static_assert(BM % 16 == 0 && BN % 8 == 0, "tile rows");
-    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kStageB];
+    static_assert(NS == 2 || (kInst % NW == 0 && (NS - 1) * kPer < 64), "whole copies per wave behind the awaited stage");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[NS * kStageB];
 
     const uint32_t M = p.M, N = p.N, K = p.K;
     const uint32_t nM = (M + BM - 1) / BM, nN = (N + BN - 1) / BN;
@@ -409,19 +295,27 @@ __device__ void gemm_nt_lines(const uint16_t *__restrict__ A, const uint16_t *__
     // offset go in the scalar offset.
     static_assert(NW % 2 == 0, "one chunk swizzle per lane for every instruction");
     const uint32_t lr = lane >> 3, lpos = lane & 7;
-    const uint32_t kBase = SPLITK ? split * (K / gridDim.y) : 0u;
+    // this block's stages: all of K's, or its split's share (near-equal
+    // whole stages)
+    const uint32_t stages = (K + BK64 - 1) / BK64;
+    const uint32_t first = SPLITK ? split * stages / gridDim.y : 0u;
+    const uint32_t nk = (SPLITK ? (split + 1) * stages / gridDim.y : stages) - first;
     const uint64_t rowB = (uint64_t)K * 2u;
-    const uint32_t bytesA = (uint32_t)min((uint64_t)(M - bm) * rowB, (uint64_t)0xffffffffu);
-    const uint32_t bytesB = (uint32_t)min((uint64_t)(N - bn) * rowB, (uint64_t)0xffffffffu);
+    const uint32_t bytesA = (uint32_t)(min(M - bm, (uint32_t)BM) * rowB);  // the host keeps a tile's rows under 2 GB
+    const uint32_t bytesB = (uint32_t)(min(N - bn, (uint32_t)BN) * rowB);
     const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(A + (uint64_t)bm * K), 0, (int)bytesA, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(B + (uint64_t)bn * K), 0, (int)bytesB, 0x00020000);
     // row 8 j + lr of an operand: chunk swizzle (4 j + lr / 2) & 7, and j is
     // odd or even with the wave (NW and kInstA even)
-    const uint32_t voff = lr * (uint32_t)rowB + ((lpos ^ (((wave & 1) * 4 + (lr >> 1)) & 7)) << 4);
+    const uint32_t chunk = lpos ^ (((wave & 1) * 4 + (lr >> 1)) & 7);
+    uint32_t voff = lr * (uint32_t)rowB + (chunk << 4);
+    // K % 64 != 0: the last stage's chunks past K read outside the resource (zeros)
+    const uint32_t voffLast = (stages - 1) * BK64 + chunk * 8 < K ? voff : 0x80000000u;
     const uint32_t rows8 = 8 * (uint32_t)rowB;  // bytes per instruction's rows
     auto issue = [&](uint32_t kt) {
-        const uint32_t kb = (kBase + kt * BK64) * 2u;
-        uint8_t *stage = smem + (kt & 1) * kStageB;
+        const uint32_t kb = (first + kt) * BK64 * 2u;
+        if (first + kt + 1 == stages) voff = voffLast;
+        uint8_t *stage = smem + (kt % NS) * kStageB;
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const uint32_t j = i * NW + wave;
@@ -431,9 +325,16 @@ __device__ void gemm_nt_lines(const uint16_t *__restrict__ A, const uint16_t *__
                                                      kb + (isA ? j : j - kInstA) * rows8, 0, 0);
         }
     };
-    // wait until only the copies of the stage after the awaited one are
-    // outstanding (this wave issues kPer or kPer - 1 of them)
-    auto wait_one_behind = [&] {
+    // wait until only the copies of the `behind` stages after the awaited
+    // one are outstanding (this wave issues kPer or kPer - 1 for a stage)
+    auto wait_behind = [&](uint32_t behind) {
+        if constexpr (NS >= 4) {
+            if (behind >= 3) return wait_vmcnt<3 * kPer>();
+        }
+        if constexpr (NS >= 3) {
+            if (behind >= 2) return wait_vmcnt<2 * kPer>();
+        }
+        if (behind == 0) return wait_vmcnt<0>();
         if (kInst % NW == 0 || wave < (uint32_t)(kInst % NW)) wait_vmcnt<kPer>();
         else wait_vmcnt<kPer - 1>();
     };
@@ -451,20 +352,16 @@ __device__ void gemm_nt_lines(const uint16_t *__restrict__ A, const uint16_t *__
     };
     // fragment mi of A / ni of B for K-16 quarter kk of stage kt
     auto fragA = [&](uint32_t kt, int kk, int mi) {
-        return frag(smem + (kt & 1) * kStageB, wm + mi * 32 + (lane & 31), kk * 2 + (lane >> 5));
+        return frag(smem + (kt % NS) * kStageB, wm + mi * 32 + (lane & 31), kk * 2 + (lane >> 5));
     };
     auto fragB = [&](uint32_t kt, int kk, int ni) {
-        return frag(smem + (kt & 1) * kStageB + BM * kRowB, wn + ni * 32 + (lane & 31), kk * 2 + (lane >> 5));
+        return frag(smem + (kt % NS) * kStageB + BM * kRowB, wn + ni * 32 + (lane & 31), kk * 2 + (lane >> 5));
     };
 
-    const uint32_t nk = (SPLITK ? K / gridDim.y : K) / BK64;
-    issue(0);
-    if (nk > 1) {
-        issue(1);
-        wait_one_behind();
-    } else {
-        wait_vmcnt<0>();
-    }
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+        if ((uint32_t)i < nk) issue(i);
+    wait_behind(min((uint32_t)(NS - 1), nk - 1));
     __builtin_amdgcn_s_barrier();
     u32x4 fa[TM], fb[TN], fb2[TN];
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -505,13 +402,15 @@ __device__ void gemm_nt_lines(const uint16_t *__restrict__ A, const uint16_t *__
         quarter(fb2, fb, kt, 2);
         quarter(fb, fb2, kt, 3);
         // this wave's reads of stage kt are issued; wait for them and for
-        // its copies of stage kt + 1 (the only ones outstanding), then the
-        // buffer of stage kt takes the copies of stage kt + 2. In the last
-        // pass the reads of "stage kt + 1" fetch a buffer no copy writes.
-        wait_vmcnt<0>();
+        // its copies of stage kt + 1 (those of up to NS - 2 later stages may
+        // be outstanding), then the buffer of stage kt takes the copies of
+        // stage kt + NS. In the last pass the reads of "stage kt + 1" fetch
+        // a buffer no copy writes.
+        if (NS == 2) wait_vmcnt<0>();
+        else wait_behind(kt + 2 < nk ? min((uint32_t)(NS - 2), nk - 2 - kt) : 0u);
         __builtin_amdgcn_s_waitcnt(0xC07F);
         __builtin_amdgcn_s_barrier();
-        if (kt + 2 < nk) issue(kt + 2);
+        if (kt + NS < nk) issue(kt + NS);
         quarter(fb2, fb, kt + 1, 0);
     }
 
@@ -535,13 +434,21 @@ __device__ void gemm_nt_lines(const uint16_t *__restrict__ A, const uint16_t *__
 }
 
 // C = sum over the gridDim.y-way split of P [splits][M][N] (f32), rounded
-// once to C's dtype; 4 elements per thread (M N % 4 == 0).
+// once to C's dtype; 4 elements per thread where M N % 4 == 0, else one.
 template <typename O>
 __device__ void gemm_splitk_reduce(const float *__restrict__ P, typename O::storage *__restrict__ C,
                                    const MatmulConstants &p, uint32_t splits) {
     const uint64_t mn = (uint64_t)p.M * p.N;
-    for (uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; i < mn;
-         i += (uint64_t)gridDim.x * blockDim.x * 4) {
+    const uint64_t id = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+    if (mn % 4 != 0) {
+        for (uint64_t i = id; i < mn; i += step) {
+            float a = P[i];
+            for (uint32_t s = 1; s < splits; ++s) a += P[s * mn + i];
+            C[i] = O::store(a);
+        }
+        return;
+    }
+    for (uint64_t i = id * 4; i < mn; i += step * 4) {
         float4 a = *reinterpret_cast<const float4 *>(P + i);
         for (uint32_t s = 1; s < splits; ++s) {
             const float4 b = *reinterpret_cast<const float4 *>(P + s * mn + i);
@@ -563,12 +470,6 @@ __device__ void gemm_splitk_reduce(const float *__restrict__ P, typename O::stor
 }  // namespace
 
 // A, B: 16-bit storage; the host requires K % 8 == 0 and 16-byte aligned A, B.
-// Tile variants: _t<BM>x<BN> on 4 (128 x 128) or 8 waves; LDS is static.
-#define GEMM_MFMA(name, T, O, BM, BN, WMN, WNN)                                                   \
-    POPCORN_KERNEL void __launch_bounds__(64 * WMN * WNN)                                         \
-        name(const uint16_t *a, const uint16_t *b, O::storage *c, MatmulConstants p) {            \
-        gemm_nt<T, O, BM, BN, WMN, WNN>(a, b, c, p);                                              \
-    }
 #define GEMM_MFMA_D(name, T, O, BM, BN, WMN, WNN)                                                 \
     POPCORN_KERNEL void __launch_bounds__(64 * WMN * WNN)                                         \
         name(const uint16_t *a, const uint16_t *b, O::storage *c, MatmulConstants p) {            \
@@ -578,6 +479,12 @@ __device__ void gemm_splitk_reduce(const float *__restrict__ P, typename O::stor
     POPCORN_KERNEL void __launch_bounds__(64 * WMN * WNN)                                         \
         name(const uint16_t *a, const uint16_t *b, O::storage *c, MatmulConstants p) {            \
         gemm_nt_lines<T, O, BM, BN, WMN, WNN>(a, b, c, p);                                        \
+    }
+// 4 stages in flight, for grids of few blocks
+#define GEMM_MFMA_F(name, T, O, BM, BN, WMN, WNN)                                                 \
+    POPCORN_KERNEL void __launch_bounds__(64 * WMN * WNN)                                         \
+        name(const uint16_t *a, const uint16_t *b, O::storage *c, MatmulConstants p) {            \
+        gemm_nt_lines<T, O, BM, BN, WMN, WNN, false, 4>(a, b, c, p);                              \
     }
 #define GEMM_MFMA_TILES(base, T, O)                          \
     GEMM_MFMA_E(base##_e256x384, T, O, 256, 384, 2, 4)       \
@@ -590,12 +497,10 @@ __device__ void gemm_splitk_reduce(const float *__restrict__ P, typename O::stor
     GEMM_MFMA_D(base##_d128x128, T, O, 128, 128, 2, 2)       \
     GEMM_MFMA_D(base##_d128x256, T, O, 128, 256, 2, 4)       \
     GEMM_MFMA_D(base##_d128x192, T, O, 128, 192, 2, 2)       \
-    GEMM_MFMA_D(base##_d256x384, T, O, 256, 384, 2, 4)       \
-    GEMM_MFMA(base##_t128x128, T, O, 128, 128, 2, 2)         \
-    GEMM_MFMA(base##_t256x128, T, O, 256, 128, 4, 2)         \
-    GEMM_MFMA(base##_t128x256, T, O, 128, 256, 2, 4)         \
-    GEMM_MFMA(base##_t256x256, T, O, 256, 256, 2, 4)         \
-    GEMM_MFMA(base##_t256x256w4, T, O, 256, 256, 2, 2)
+    GEMM_MFMA_D(base##_d256x384, T, O, 256, 384, 2, 4)         \
+    GEMM_MFMA_F(base##_f64x64, T, O, 64, 64, 2, 2)           \
+    GEMM_MFMA_F(base##_f128x64, T, O, 128, 64, 2, 2)         \
+    GEMM_MFMA_F(base##_f128x128, T, O, 128, 128, 2, 2)
 
 using pk::BF16;
 using pk::F16;
@@ -606,7 +511,6 @@ GEMM_MFMA_TILES(matmul_mfma_f16_f16_f32, F16, F32)
 GEMM_MFMA_TILES(matmul_mfma_bf16_bf16_bf16, BF16, BF16)
 GEMM_MFMA_TILES(matmul_mfma_bf16_bf16_f32, BF16, F32)
 
-// Split-K forms of the 256 x 384 tile (f32 partials) and the reduction.
 // B^T for a Matmul whose 16-bit B is [K, N] (not transposed): a block moves
 // a 64 x 64 tile through LDS (66-element rows: a column read touches 32
 // distinct banks). Whole tiles of 8-aligned shapes move as 16-byte runs (a
@@ -662,6 +566,7 @@ POPCORN_KERNEL void __launch_bounds__(256) transpose2d_b16(const uint16_t *in, u
     transpose2d_run(in, out, p);
 }
 
+// Split-K forms (f32 partials) and the reduction.
 #define GEMM_MFMA_SPLITK(name, T)                                                                 \
     POPCORN_KERNEL void __launch_bounds__(512)                                                    \
         name(const uint16_t *a, const uint16_t *b, float *partial, MatmulConstants p) {          \
@@ -672,15 +577,22 @@ POPCORN_KERNEL void __launch_bounds__(256) transpose2d_b16(const uint16_t *in, u
         name(const float *partial, O::storage *c, MatmulConstants p, uint32_t splits) {                \
         gemm_splitk_reduce<O>(partial, c, p, splits);                                                  \
     }
-#define GEMM_MFMA_SPLITK_E(name, T)                                                               \
-    POPCORN_KERNEL void __launch_bounds__(512)                                                    \
+#define GEMM_MFMA_SPLITK_E(name, T, BM, BN, WMN, WNN, NS)                                         \
+    POPCORN_KERNEL void __launch_bounds__(64 * WMN * WNN)                                         \
         name(const uint16_t *a, const uint16_t *b, float *partial, MatmulConstants p) {          \
-        gemm_nt_lines<T, F32, 256, 384, 2, 4, true>(a, b, nullptr, p, partial);                   \
+        gemm_nt_lines<T, F32, BM, BN, WMN, WNN, true, NS>(a, b, nullptr, p, partial);             \
     }
-GEMM_MFMA_SPLITK(matmul_mfma_f16_splitk_d256x384, F16)
-GEMM_MFMA_SPLITK(matmul_mfma_bf16_splitk_d256x384, BF16)
-GEMM_MFMA_SPLITK_E(matmul_mfma_f16_splitk_e256x384, F16)
-GEMM_MFMA_SPLITK_E(matmul_mfma_bf16_splitk_e256x384, BF16)
+#define GEMM_MFMA_SPLITK_TILES(base, T)                              \
+    GEMM_MFMA_SPLITK(base##_d256x384, T)                             \
+    GEMM_MFMA_SPLITK_E(base##_e256x384, T, 256, 384, 2, 4, 2)        \
+    GEMM_MFMA_SPLITK_E(base##_e256x256, T, 256, 256, 2, 4, 2)        \
+    GEMM_MFMA_SPLITK_E(base##_e128x128, T, 128, 128, 2, 2, 2)        \
+    GEMM_MFMA_SPLITK_E(base##_f64x64, T, 64, 64, 2, 2, 4)            \
+    GEMM_MFMA_SPLITK_E(base##_f128x64, T, 128, 64, 2, 2, 4)          \
+    GEMM_MFMA_SPLITK_E(base##_f128x128, T, 128, 128, 2, 2, 4)
+
+GEMM_MFMA_SPLITK_TILES(matmul_mfma_f16_splitk, F16)
+GEMM_MFMA_SPLITK_TILES(matmul_mfma_bf16_splitk, BF16)
 GEMM_SPLITK_REDUCE(matmul_splitk_reduce_f16, F16)
 GEMM_SPLITK_REDUCE(matmul_splitk_reduce_bf16, BF16)
 GEMM_SPLITK_REDUCE(matmul_splitk_reduce_f32, F32)

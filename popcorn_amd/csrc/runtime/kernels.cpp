@@ -690,11 +690,13 @@ struct GemmTile {
     const char *suffix;
 };
 
-// "d" tiles copy operands global -> LDS directly (4 stages of K 32); they
-// need K % 32 == 0. Their "e" forms copy whole 128-byte lines (2 stages of
-// K 64, buffer loads whose byte offsets stay below 2^31 over a tile's rows);
-// they need K % 64 == 0 and take every such shape.
-bool gemmLinesFit(int64_t k, int bn) { return k % 64 == 0 && (int64_t)(bn + 16) * k * 2 < (int64_t{1} << 31); }
+// "e" and "f" tiles copy whole 128-byte lines global -> LDS (stages of K 64,
+// the last one's chunks past K reading zeros; 2 stages, or 4 in the "f"
+// forms, by buffer loads whose byte offsets stay below 2^31 over a tile's
+// rows). "d" tiles copy 64-byte rows (4 stages of K 32) and keep K % 64 ==
+// 32, which they fill in whole stages.
+bool gemmOffsetsFit(int64_t k, int bn) { return (int64_t)(bn + 16) * k * 2 < (int64_t{1} << 31); }
+bool gemmLinesFit(int64_t k, int bn) { return k % 64 != 32 && gemmOffsetsFit(k, bn); }
 
 // The whole-line tiles are chosen by a score: the share of the CU slots
 // their grid keeps busy over its rounds (two blocks per CU for the tiles
@@ -736,6 +738,63 @@ const ScoredTile &bestLineTile(int64_t m, int64_t n) {
     return *best;
 }
 
+// Small grids: products of at least 2^29 multiply-adds (below that a product
+// is mostly launch and one 128 x 128 pass keeps it at one launch) whose
+// 128 x 128 tiles give no more than two per CU. There the CUs, not the tile's
+// rate, set the time, so the plan chooses a tile and a number of K splits
+// together, by the time that a block's stages take:
+//   rounds of blocks x (stages per block x us per stage + us per block)
+//   + for a split, the reduction's launch and its partials' trip through HBM,
+// with us per stage from a fit over 68 shapes (bf16, m 65-1800, the
+// projections of the Gemma shapes and odd sizes, 1 to 16 splits; the plan's
+// pick is on average 2% slower than the fastest of every tile and split, 20%
+// at worst). M 137, K 9216, N 2304: 85.9 us on 36 tiles of 128 x 128, 19.8
+// on 128 x 128 tiles and 7 splits; M 1000, K 9216, N 2304: 91.5 -> 51; M 1000,
+// K 2304, N 1024: 25.6 -> 13.3 on 64 x 64 tiles. With more than two tiles per
+// CU the score above is as good (M 1000, K 2304, N 9216: 48.8 both ways).
+struct SmallTile {
+    GemmTile tile;
+    int blocksPerCU;
+    double alone, full, block;  // us per stage with one block per CU, with the CU full, and us per block
+};
+const SmallTile kSmallTiles[] = {{{64, 64, 256, "f64x64"}, 2, 0.313, 0.500, 0.2},
+                                 {{128, 64, 256, "f128x64"}, 1, 0.402, 0.407, 0.8},
+                                 {{128, 128, 256, "e128x128"}, 2, 0.790, 1.209, 0.6},
+                                 {{128, 128, 256, "f128x128"}, 1, 0.604, 0.662, 1.6},
+                                 {{256, 256, 512, "e256x256"}, 1, 1.620, 1.932, 0.4}};
+
+bool gemmSmallGrid(int64_t m, int64_t n, int64_t k) {
+    return (double)m * (double)n * (double)k >= 0x1p29 && cdiv(m, 128) * cdiv(n, 128) <= 2 * (int64_t)deviceCUs() &&
+           gemmOffsetsFit(k, 384);
+}
+
+struct GemmPlan {
+    GemmTile tile;
+    int64_t splits;
+};
+
+GemmPlan gemmSmallPlan(int64_t m, int64_t n, int64_t k, bool maySplit) {
+    const int64_t cus = deviceCUs(), stages = cdiv(k, 64);
+    GemmPlan best{kSmallTiles[0].tile, 1};
+    double bestUs = 1e30;
+    for (const SmallTile &t : kSmallTiles) {
+        const int64_t tiles = cdiv(m, t.tile.bm) * cdiv(n, t.tile.bn);
+        // a split takes at least 4 stages; more than 16 were never the fastest
+        for (int64_t s = 1; s <= 16 && (s == 1 || (maySplit && stages / s >= 4)); ++s) {
+            const int64_t slots = cus * t.blocksPerCU, rounds = tiles * s / slots, rest = tiles * s % slots;
+            const double per = (double)cdiv(stages, s), over = std::max(0.0, (double)rest / (double)cus - 1.0);
+            double us = (double)rounds * (per * t.full + t.block);
+            if (rest) us += per * (t.alone + (t.full - t.alone) * over) + t.block;
+            if (s > 1) us += 4.3 + 0.14 * 8e-6 * (double)s * (double)m * (double)n;
+            if (us < bestUs) {
+                bestUs = us;
+                best = GemmPlan{t.tile, s};
+            }
+        }
+    }
+    return best;
+}
+
 GemmTile gemmTileForm(int64_t m, int64_t n, int64_t k);
 GemmTile gemmTile(int64_t m, int64_t n, int64_t k) {
     if (!std::getenv("POPCORN_GEMM_TILE") && gemmLinesFit(k, 384)) return bestLineTile(m, n).tile;
@@ -743,51 +802,45 @@ GemmTile gemmTile(int64_t m, int64_t n, int64_t k) {
 }
 
 GemmTile gemmTileForm(int64_t m, int64_t n, int64_t k) {
-    static const GemmTile tiles[] = {{256, 256, 512, "t256x256"}, {256, 256, 256, "t256x256w4"},
-                                     {256, 128, 512, "t256x128"}, {128, 256, 512, "t128x256"},
-                                     {128, 128, 256, "t128x128"}, {256, 256, 512, "d256x256"},
-                                     {128, 128, 256, "d128x128"}, {128, 256, 512, "d128x256"},
-                                     {128, 192, 256, "d128x192"}, {256, 384, 512, "d256x384"},
-                                     {256, 256, 512, "e256x256"}, {128, 128, 256, "e128x128"},
-                                     {128, 256, 512, "e128x256"}, {128, 192, 256, "e128x192"},
-                                     {256, 384, 512, "e256x384"}, {256, 288, 768, "e256x288"}};
-    if (const char *e = std::getenv("POPCORN_GEMM_TILE")) {  // tuning override, e.g. "t256x128"
+    static const GemmTile tiles[] = {{256, 256, 512, "d256x256"}, {128, 128, 256, "d128x128"},
+                                     {128, 256, 512, "d128x256"}, {128, 192, 256, "d128x192"},
+                                     {256, 384, 512, "d256x384"}, {256, 256, 512, "e256x256"},
+                                     {128, 128, 256, "e128x128"}, {128, 256, 512, "e128x256"},
+                                     {128, 192, 256, "e128x192"}, {256, 384, 512, "e256x384"},
+                                     {256, 288, 768, "e256x288"}, {64, 64, 256, "f64x64"},
+                                     {128, 64, 256, "f128x64"},   {128, 128, 256, "f128x128"}};
+    if (const char *e = std::getenv("POPCORN_GEMM_TILE")) {  // tuning override, e.g. "e128x192"
         for (const GemmTile &t : tiles)
-            if (std::string(t.suffix) == e && (t.suffix[0] != 'd' || k % 32 == 0) && (t.suffix[0] != 'e' || gemmLinesFit(k, t.bn)))
-                return t;
+            if (std::string(t.suffix) == e && (t.suffix[0] == 'd' ? k % 32 == 0 : gemmOffsetsFit(k, std::max(t.bm, t.bn)))) return t;
     }
+    if (k % 32 != 0) return tiles[6];  // an override that does not fit
     // 256 x 256 on 8 waves reuses each LDS stage for twice the MFMA work of
     // 128 x 128 but runs one block per CU, so it only pays when the tiles
     // fill the CUs several times over; below that the 128 x 128 grid (two
-    // blocks per CU) balances better. The direct-to-LDS forms beat the
-    // register-staged ones on every config-5 shape (f16, M 2048; us):
-    //                      d256  d128  t256  t128
-    //   QKV  N 9216  K 3072   177   162   203   186
-    //   gate N 24576 K 3072   319   422   375   431
-    //   down N 3072  K 24576  589   430   712   485
-    const bool big = cdiv(m, 256) * cdiv(n, 256) >= 3 * deviceCUs();
-    if (k % 32 == 0) {
-        // 256 x 384 (8 waves of 128 x 96: 7 fragment reads per 12 MFMAs) when
-        // its grid keeps at least 70% of the CUs busy in every round
-        // (config-5 QKV, 192 tiles: 136 -> 127 us; gate and up, 512 tiles:
-        // 294-303 -> 284-288 us)
-        const int64_t cus = deviceCUs();
-        const int64_t t384 = cdiv(m, 256) * cdiv(n, 384);
-        if (t384 * 10 >= cus * 7 && t384 * 10 >= cdiv(t384, cus) * cus * 7) return tiles[9];
-        if (big) return tiles[5];
-        // 128 x 192 tiles when their grid is whole rounds of one tile per CU
-        // (config-5 QKV, N 9216: 768 tiles, 155 -> 135 us; down, N 3072:
-        // 256 tiles, 397 -> 352 us)
-        const int64_t t192 = cdiv(m, 128) * cdiv(n, 192);
-        if (n % 192 == 0 && t192 % deviceCUs() == 0) return tiles[8];
-        // a 128 x 128 grid between one and two tiles per CU leaves half the
-        // CUs with a second tile; one 128 x 256 tile per CU (8 waves) ends
-        // sooner (config-5 down: 379 against 423 us before 128 x 192 took it)
-        const int64_t t128 = cdiv(m, 128) * cdiv(n, 128);
-        if (t128 > deviceCUs() && t128 < 2 * (int64_t)deviceCUs() && n >= 256) return tiles[7];
-        return tiles[6];
-    }
-    return big ? tiles[0] : tiles[4];
+    // blocks per CU) balances better (config 5, f16, M 2048; us):
+    //                      d256  d128
+    //   QKV  N 9216  K 3072   177   162
+    //   gate N 24576 K 3072   319   422
+    //   down N 3072  K 24576  589   430
+    // 256 x 384 (8 waves of 128 x 96: 7 fragment reads per 12 MFMAs) when
+    // its grid keeps at least 70% of the CUs busy in every round
+    // (config-5 QKV, 192 tiles: 136 -> 127 us; gate and up, 512 tiles:
+    // 294-303 -> 284-288 us)
+    const int64_t cus = deviceCUs();
+    const int64_t t384 = cdiv(m, 256) * cdiv(n, 384);
+    if (t384 * 10 >= cus * 7 && t384 * 10 >= cdiv(t384, cus) * cus * 7) return tiles[4];
+    if (cdiv(m, 256) * cdiv(n, 256) >= 3 * cus) return tiles[0];
+    // 128 x 192 tiles when their grid is whole rounds of one tile per CU
+    // (config-5 QKV, N 9216: 768 tiles, 155 -> 135 us; down, N 3072:
+    // 256 tiles, 397 -> 352 us)
+    const int64_t t192 = cdiv(m, 128) * cdiv(n, 192);
+    if (n % 192 == 0 && t192 % cus == 0) return tiles[3];
+    // a 128 x 128 grid between one and two tiles per CU leaves half the
+    // CUs with a second tile; one 128 x 256 tile per CU (8 waves) ends
+    // sooner (config-5 down: 379 against 423 us before 128 x 192 took it)
+    const int64_t t128 = cdiv(m, 128) * cdiv(n, 128);
+    if (t128 > cus && t128 < 2 * cus && n >= 256) return tiles[2];
+    return tiles[1];
 }
 
 // Split-K for a GEMM whose 256 x 384 tiles are too few to fill the CUs:
@@ -815,19 +868,21 @@ int64_t gemmSplitK(int64_t m, int64_t n, int64_t k) {
 }
 
 // The split-K GEMM: f32 partial products per split in scratch, then one
-// pass that sums them and rounds to C's dtype.
+// pass that sums them and rounds to C's dtype. Without scratch (none to be
+// had, or a capture that would have to allocate it) the whole product runs on
+// unsplit tiles.
 class SplitKMatmulKernel : public Kernel {
 public:
-    SplitKMatmulKernel(const Tensor &a, const Tensor &b, const Tensor &c, int64_t m, int64_t k, int64_t n, int64_t splits)
-        : a_(a), b_(b), c_(c), m_(m), k_(k), n_(n), splits_(splits) {}
+    SplitKMatmulKernel(const Tensor &a, const Tensor &b, const Tensor &c, int64_t m, int64_t k, int64_t n, GemmPlan plan)
+        : a_(a), b_(b), c_(c), m_(m), k_(k), n_(n), splits_(plan.splits), tile_(plan.tile) {}
     std::vector<Binding> tensors() const override { return {{a_, kRead}, {b_, kRead}, {c_, kWrite}}; }
     std::string describe() const override { return mainName() + "," + reduceName(); }
     void encode(KernelCommandEncoder &enc) const override {
         MatmulConstants mc{(uint32_t)m_, (uint32_t)k_, (uint32_t)n_, 1u};
-        enc.withTemporaryTensor(ScratchSpec{{splits_ * m_, n_}, DataType::f32}, [&](Tensor part) {
+        const bool done = enc.tryTemporaryTensor(ScratchSpec{{splits_ * m_, n_}, DataType::f32}, [&](Tensor part) {
             DispatchSize ds;
-            ds.grid = dim3((unsigned)(cdiv(m_, 256) * cdiv(n_, 384)), (unsigned)splits_, 1);
-            ds.block = dim3(512, 1, 1);
+            ds.grid = dim3((unsigned)(cdiv(m_, tile_.bm) * cdiv(n_, tile_.bn)), (unsigned)splits_, 1);
+            ds.block = dim3((unsigned)tile_.threads, 1, 1);
             FixedDispatch s1(mainName(), {{a_, kRead}, {b_, kRead}, {part, kWrite}}, {bytesOf(mc)}, ds);
             enc.dispatch(s1);
             const uint32_t splits = (uint32_t)splits_;
@@ -835,17 +890,21 @@ public:
             FixedDispatch s2(reduceName(), {{part, kRead}, {c_, kWrite}}, {bytesOf(mc), bytesOf(splits)}, grid1(blocks, kBlock));
             enc.dispatch(s2);
         });
+        if (done) return;
+        const GemmTile tile = gemmTile(m_, n_, k_);
+        FixedDispatch whole(std::string("matmul_mfma_") + tag(a_.dataType) + "_" + tag(a_.dataType) + "_" +
+                                tag(c_.dataType) + "_" + tile.suffix,
+                            {{a_, kRead}, {b_, kRead}, {c_, kWrite}}, {bytesOf(mc)},
+                            grid1(cdiv(m_, tile.bm) * cdiv(n_, tile.bn), tile.threads));
+        enc.dispatch(whole);
     }
 
 private:
-    std::string mainName() const {
-        // each split's K a whole number of 64-deep stages; offsets span the full rows
-        const bool lines = gemmLinesFit(k_, 384) && k_ % (64 * splits_) == 0;
-        return std::string("matmul_mfma_") + tag(a_.dataType) + (lines ? "_splitk_e256x384" : "_splitk_d256x384");
-    }
+    std::string mainName() const { return std::string("matmul_mfma_") + tag(a_.dataType) + "_splitk_" + tile_.suffix; }
     std::string reduceName() const { return std::string("matmul_splitk_reduce_") + tag(c_.dataType); }
     Tensor a_, b_, c_;
     int64_t m_, k_, n_, splits_;
+    GemmTile tile_;
 };
 
 constexpr int64_t kMaxStagedK = 16384;  // x staged as f32 in 64 KB of LDS
@@ -949,15 +1008,28 @@ std::unique_ptr<Kernel> makeMatmul(const Tensor &a, const Tensor &b, const Tenso
                 return std::make_unique<FixedDispatch>(fn, binds, std::vector<std::vector<uint8_t>>{bytesOf(mc)},
                                                        grid1(blocks, (int)(64 * w)));
             }
-            // the split-K reduction stores 4 results of C at a time
-            if (const int64_t splits = aligned16(c.data) ? gemmSplitK(m, n, k) : 0)
-                return std::make_unique<SplitKMatmulKernel>(a, b, c, m, k, n, splits);
-            MatmulConstants mc{(uint32_t)m, (uint32_t)k, (uint32_t)n, 1u};
-            const GemmTile tile = gemmTile(m, n, k);
-            const std::string fn =
-                std::string("matmul_mfma_") + tag(t) + "_" + tag(t) + "_" + tag(c.dataType) + "_" + tile.suffix;
-            return std::make_unique<FixedDispatch>(fn, binds, std::vector<std::vector<uint8_t>>{bytesOf(mc)},
-                                                   grid1(cdiv(m, tile.bm) * cdiv(n, tile.bn), tile.threads));
+            // (rows too long for 32-bit offsets over a tile that the 64-byte-row
+            // tiles do not take either go to the SIMT tiles below)
+            if (k % 32 == 0 || gemmOffsetsFit(k, 384)) {
+                // the split-K reduction stores 4 results of C at a time
+                if (const int64_t splits = aligned16(c.data) ? gemmSplitK(m, n, k) : 0) {
+                    // each split's K a whole number of 64-deep stages
+                    const bool lines = gemmLinesFit(k, 384) && k % (64 * splits) == 0;
+                    return std::make_unique<SplitKMatmulKernel>(
+                        a, b, c, m, k, n, GemmPlan{{256, 384, 512, lines ? "e256x384" : "d256x384"}, splits});
+                }
+                MatmulConstants mc{(uint32_t)m, (uint32_t)k, (uint32_t)n, 1u};
+                GemmTile tile = gemmTile(m, n, k);
+                if (!std::getenv("POPCORN_GEMM_TILE") && gemmSmallGrid(m, n, k)) {
+                    const GemmPlan plan = gemmSmallPlan(m, n, k, aligned16(c.data));
+                    if (plan.splits > 1) return std::make_unique<SplitKMatmulKernel>(a, b, c, m, k, n, plan);
+                    tile = plan.tile;
+                }
+                const std::string fn =
+                    std::string("matmul_mfma_") + tag(t) + "_" + tag(t) + "_" + tag(c.dataType) + "_" + tile.suffix;
+                return std::make_unique<FixedDispatch>(fn, binds, std::vector<std::vector<uint8_t>>{bytesOf(mc)},
+                                                       grid1(cdiv(m, tile.bm) * cdiv(n, tile.bn), tile.threads));
+            }
         }
     }
     // m > 1 with f32 output and an f32 operand (the reference's MPP f32

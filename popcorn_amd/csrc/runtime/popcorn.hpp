@@ -121,6 +121,9 @@ public:
     virtual ~KernelScratchAllocator() = default;
     virtual KernelTemporaryBuffer borrowTemporaryBuffer(size_t length) = 0;
     virtual void releaseTemporaryBuffer(const KernelTemporaryBuffer &) {}
+    // Whether a borrow of `length` bytes would be served from memory already
+    // held (false where that is not known).
+    virtual bool holds(size_t length) const { return false; }
 };
 
 // Best-fit pool over hipMalloc'd buffers for one stream (the GemmaCLI
@@ -130,6 +133,7 @@ public:
     ~ScratchPool() override;
     KernelTemporaryBuffer borrowTemporaryBuffer(size_t length) override;
     void releaseTemporaryBuffer(const KernelTemporaryBuffer &t) override;
+    bool holds(size_t length) const override;
     size_t bytes() const;
 
 private:
@@ -267,15 +271,23 @@ public:
 
     template <typename F>
     void withTemporaryTensor(const ScratchSpec &spec, F &&body) {
-        KernelTemporaryBuffer t = scratch_.borrowTemporaryBuffer(spec.byteCount());
-        ++scratchBorrows_;
-        if (t.wasReused) accessByBuffer_[t.buffer] |= kWrite;
-        struct Release {
-            KernelScratchAllocator &s;
-            KernelTemporaryBuffer t;
-            ~Release() { s.releaseTemporaryBuffer(t); }
-        } release{scratch_, t};
-        body(Tensor(t.buffer, Shape(spec.shape), spec.dataType));
+        withBuffer(scratch_.borrowTemporaryBuffer(spec.byteCount()), spec, body);
+    }
+
+    // The same for work that can also be done without the scratch: false, and
+    // nothing done, where the allocator has none to give or, while the stream
+    // is being captured, would have to allocate it.
+    template <typename F>
+    bool tryTemporaryTensor(const ScratchSpec &spec, F &&body) {
+        if (capturing() && !scratch_.holds(spec.byteCount())) return false;
+        KernelTemporaryBuffer t;
+        try {
+            t = scratch_.borrowTemporaryBuffer(spec.byteCount());
+        } catch (const Error &) {
+            return false;
+        }
+        withBuffer(t, spec, body);
+        return true;
     }
 
     KernelLibrary &library() { return library_; }
@@ -292,6 +304,18 @@ public:
 
 
 private:
+    template <typename F>
+    void withBuffer(const KernelTemporaryBuffer &t, const ScratchSpec &spec, F &&body) {
+        ++scratchBorrows_;
+        if (t.wasReused) accessByBuffer_[t.buffer] |= kWrite;
+        struct Release {
+            KernelScratchAllocator &s;
+            KernelTemporaryBuffer t;
+            ~Release() { s.releaseTemporaryBuffer(t); }
+        } release{scratch_, t};
+        body(Tensor(t.buffer, Shape(spec.shape), spec.dataType));
+    }
+    bool capturing() const;
     bool needsBarrier(const std::vector<Binding> &bindings) const;
     void recordAccesses(const std::vector<Binding> &bindings);
 

@@ -138,6 +138,11 @@ void ScratchPool::releaseTemporaryBuffer(const KernelTemporaryBuffer &t) {
     if (it != all_.end()) free_.emplace(it->second, t.buffer);
 }
 
+bool ScratchPool::holds(size_t length) const {
+    std::lock_guard<std::mutex> g(mu_);
+    return free_.lower_bound(std::max<size_t>(length, 1)) != free_.end();
+}
+
 size_t ScratchPool::bytes() const {
     std::lock_guard<std::mutex> g(mu_);
     return bytes_;
@@ -253,6 +258,16 @@ void DispatchKernel::encode(KernelCommandEncoder &encoder) const { encoder.dispa
 
 KernelCommandEncoder::KernelCommandEncoder(KernelLibrary &library, hipStream_t stream, KernelScratchAllocator &scratch)
     : library_(library), stream_(stream), scratch_(scratch) {}
+
+bool KernelCommandEncoder::capturing() const {
+    if (!stream_) return false;  // the default stream cannot be captured
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream_, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
 
 // KernelCommandEncoder.swift:155-162: a binding conflicts with an earlier
 // access when either side writes.
