@@ -134,9 +134,13 @@ typedef struct {
  *              blocks may sit on XCDs whose L2 caches are not coherent.
  *              pairFlags (u64) holds the abort word at index 0 and the flag
  *              of split tile t at index 1 + t; all start at 0;
+ *              3 (splitFrom 0): every tile's key steps run as near-equal
+ *              runs of at most ticketLo steps, one block each, ticketHi
+ *              blocks per head (the tiles' runs in all), the last tile's
+ *              first; a tile of several runs goes to the split-merge kernel;
  *              The _d512 kernels (64 query rows per block, 256 threads)
  *              run every tile whole whatever splitFrom and pairTiles say;
- *   ticketLo, ticketHi  pairTiles 2: the 64-bit value (neither 0 nor
+ *   ticketLo, ticketHi  pairTiles 3: as above; 2: the 64-bit value (neither 0 nor
  *              ~0) the first block sets its flag to, by compare-and-swap
  *              from 0, distinct per launch; the merging block resets the
  *              flag to 0. A merging block that gives up (0.2 s, or a flag

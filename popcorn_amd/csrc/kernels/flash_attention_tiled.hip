@@ -165,11 +165,22 @@ __device__ inline uint32_t fa_steps(const TiledFlashAttentionConstants &p, uint3
 // their key steps and blocks take the items heaviest first (the larger of
 // the next split half and the next whole tile), the (batch, head) index
 // varying fastest, so the longest items start first on every CU.
+// pairTiles 3 (runs): every tile's key steps are cut into near-equal runs of
+// at most ticketLo steps, one block each, the heaviest tiles first; a tile of
+// one run is written whole, the others' runs are merged by the merge kernel.
+// For calls of fewer tiles than CUs and many keys (a chunk of a prompt behind
+// its cache): 8 heads, 500 rows, 8692 keys, Hd 256 have 32 tiles of 257-272
+// steps, which ran on 32 of the 256 CUs.
 struct FaWork {
     uint32_t bh, n;
     uint32_t qt[2], lo[2], hi[2], part[2];
+    uint32_t slot;  // partial-state tile of a split item that is not a merged pair's
     bool split[2];
 };
+
+__device__ inline uint32_t fa_runs(const TiledFlashAttentionConstants &p, uint32_t qt) {
+    return max((fa_steps(p, qt) + p.ticketLo - 1) / p.ticketLo, 1u);
+}
 
 __device__ inline FaWork fa_work(const TiledFlashAttentionConstants &p, uint32_t bq = BQ, bool whole = false) {
     const uint32_t BH = p.B * p.Nq, nQT = p.qTilesPerHead;
@@ -180,6 +191,20 @@ __device__ inline FaWork fa_work(const TiledFlashAttentionConstants &p, uint32_t
     if (whole || p.splitFrom >= nQT) {
         w.qt[0] = nQT - 1 - rank;
         w.hi[0] = fa_steps(p, w.qt[0], bq);
+        return w;
+    }
+    if (p.pairTiles == 3u) {
+        uint32_t qt = nQT - 1, first = 0, runs = fa_runs(p, qt);
+        while (rank - first >= runs && qt > 0) {
+            first += runs;
+            runs = fa_runs(p, --qt);
+        }
+        const uint32_t n = fa_steps(p, qt, bq), run = rank - first;
+        w.qt[0] = qt;
+        w.lo[0] = n * run / runs;
+        w.hi[0] = n * (run + 1) / runs;
+        w.split[0] = runs > 1;
+        w.slot = w.bh * p.ticketHi + rank;
         return w;
     }
     if (!p.pairTiles) {
@@ -195,6 +220,7 @@ __device__ inline FaWork fa_work(const TiledFlashAttentionConstants &p, uint32_t
                 w.part[0] = takeSplit ? 2u - halves : 0u;
                 w.lo[0] = takeSplit && w.part[0] == 1u ? half : 0u;
                 w.hi[0] = takeSplit && w.part[0] == 0u ? half : n;
+                w.slot = (w.bh * (nQT - sf) + (qt - sf)) * 2u + w.part[0];
                 break;
             }
             if (takeSplit) {
@@ -217,6 +243,7 @@ __device__ inline FaWork fa_work(const TiledFlashAttentionConstants &p, uint32_t
     const uint32_t i = rank >> 1, a = i, bt = nQT - 1 - i;
     const uint32_t sa = fa_steps(p, a, bq), sb = fa_steps(p, bt, bq);
     const uint32_t x = (sa + sb + 1) / 2 - sa;
+    w.slot = (w.bh * (nQT - p.splitFrom) + (bt - p.splitFrom)) * 2u + (rank & 1u);
     if ((rank & 1u) == 0u && p.pairTiles == 2u) {
         // merged in the kernel: the partner's first steps come first, so
         // their partial state is published long before the second block
@@ -610,8 +637,7 @@ __device__ void fa_tiled(const uint16_t *__restrict__ Q, const uint16_t *__restr
             // a row past Sq (ragged last tile) writes nothing
         } else if (work.split[w]) {
             // unnormalised O (f32), and m (log2 units) and l, of this half
-            const uint32_t tile = (bh * (p.qTilesPerHead - p.splitFrom) + (qt - p.splitFrom)) * 2u + work.part[w];
-            const uint64_t row = (uint64_t)tile * BQ + wave * 32 + c32;
+            const uint64_t row = (uint64_t)work.slot * BQ + wave * 32 + c32;
             float *prow = pO + row * HD;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
@@ -978,8 +1004,7 @@ __device__ void fa_tiled16(const uint16_t *__restrict__ Q, const uint16_t *__res
         } else if (myq >= p.Sq) {
             // a row past Sq (ragged last tile) writes nothing
         } else if (kSplits && work.split[w]) {
-            const uint32_t tile = (bh * (p.qTilesPerHead - p.splitFrom) + (qt - p.splitFrom)) * 2u + work.part[w];
-            const uint64_t row = (uint64_t)tile * BQ16 + wave * 16 + c16;
+            const uint64_t row = (uint64_t)work.slot * BQ16 + wave * 16 + c16;
             float *prow = pO + row * HD;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
@@ -1196,42 +1221,70 @@ __device__ void fa_tiled_f32(const float *__restrict__ Q, const float *__restric
     }
 }
 
-// Combine of a split tile's two halves (maxima in log2 units):
-//   M = max(m0, m1), w_i = 2^(m_i - M) (0 for a half with no visible key),
-//   O = (w0 O0 + w1 O1) / (w0 l0 + w1 l1),
-// the log-sum-exp combine of FlashDecoding.metal:202-227 for two partitions.
-// One block per 16 rows of a split tile; a thread takes 4 dims of a row.
-constexpr int kMergeRows = 16;
-
+// Combine of a split tile's parts (maxima in log2 units):
+//   M = max m_i, w_i = 2^(m_i - M) (0 for a part with no visible key),
+//   O = (sum w_i O_i) / (sum w_i l_i),
+// the log-sum-exp combine of FlashDecoding.metal:202-227. HD / 4 lanes take a
+// row, 4 dims each, 1024 / HD rows a block. Bound by the stream of the
+// partials and the round trips behind it: lane i of a row's group loads part
+// i's (m, l), so the weights cost one, and the O loads of 8 parts are in
+// flight together. (Each thread walking the
+// parts' m in turn and one block per 16 rows made a call of 48 rows x 16000
+// keys, 8 heads, Hd 256, f16 60.7 us instead of 36.7.)
 template <typename O, int HD>
 __device__ void fa_split_merge(const float *__restrict__ pO, const float *__restrict__ pML,
                                typename O::storage *__restrict__ out, const TiledFlashAttentionConstants &p) {
-    const uint32_t nSplit = p.qTilesPerHead - p.splitFrom;
-    const uint32_t tile = blockIdx.x / (BQ / kMergeRows);  // bh * nSplit + (qt - splitFrom)
-    const uint32_t r0 = blockIdx.x % (BQ / kMergeRows) * kMergeRows;
-    const uint32_t bh = tile / nSplit, qt = p.splitFrom + tile % nSplit;
-    constexpr uint32_t kPerRow = HD / 4;
-    for (uint32_t idx = threadIdx.x; idx < (uint32_t)kMergeRows * kPerRow; idx += blockDim.x) {
-        const uint32_t r = r0 + idx / kPerRow, d = (idx % kPerRow) * 4;
-        const uint32_t q = qt * BQ + r;
-        if (q >= p.Sq) continue;
-        const uint64_t row0 = (uint64_t)tile * 2 * BQ + r, row1 = row0 + BQ;
-        const float2 ml0 = *reinterpret_cast<const float2 *>(pML + 2 * row0);
-        const float2 ml1 = *reinterpret_cast<const float2 *>(pML + 2 * row1);
-        const float M = fmaxf(ml0.x, ml1.x);
-        const float w0 = ml0.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml0.x - M);
-        const float w1 = ml1.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml1.x - M);
-        const float L = w0 * ml0.y + w1 * ml1.y;
-        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-        const float4 a = *reinterpret_cast<const float4 *>(pO + row0 * HD + d);
-        const float4 c = *reinterpret_cast<const float4 *>(pO + row1 * HD + d);
-        if (d >= p.Hd) continue;  // padding dims of a kernel compiled for HD > Hd
-        typename O::storage *orow = out + ((uint64_t)bh * p.Sq + q) * p.Hd + d;
-        orow[0] = O::store((w0 * a.x + w1 * c.x) * inv);
-        orow[1] = O::store((w0 * a.y + w1 * c.y) * inv);
-        orow[2] = O::store((w0 * a.z + w1 * c.z) * inv);
-        orow[3] = O::store((w0 * a.w + w1 * c.w) * inv);
+    constexpr uint32_t kLanes = HD / 4, kRows = 256 / kLanes;  // lanes per row, rows per block
+    const bool runMode = p.pairTiles == 3u;
+    const uint32_t from = runMode ? 0u : p.splitFrom, perHead = p.qTilesPerHead - from;
+    const uint32_t tile = blockIdx.x / (BQ / kRows);  // bh * perHead + (qt - from)
+    const uint32_t bh = tile / perHead, qt = from + tile % perHead;
+    uint32_t parts = 2, slot = tile * 2;
+    if (runMode) {
+        parts = fa_runs(p, qt);
+        if (parts == 1u) return;  // written whole by its block
+        slot = bh * p.ticketHi;
+        for (uint32_t t = p.qTilesPerHead - 1; t > qt; --t) slot += fa_runs(p, t);
     }
+    const uint32_t lane = threadIdx.x % kLanes, d = lane * 4;
+    const uint32_t r = blockIdx.x % (BQ / kRows) * kRows + threadIdx.x / kLanes;
+    const uint32_t q = qt * BQ + r;
+    if (q >= p.Sq) return;  // ragged tile (a row's lanes leave together)
+    const float2 *ml = reinterpret_cast<const float2 *>(pML) + (uint64_t)slot * BQ + r;
+    const float *po = pO + ((uint64_t)slot * BQ + r) * HD + d;
+    float M = -INFINITY;
+    for (uint32_t i = lane; i < parts; i += kLanes) M = fmaxf(M, ml[(uint64_t)i * BQ].x);
+    M = pk::group_max<kLanes>(M);
+    float L = 0.0f;
+    float4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t i0 = 0; i0 < parts; i0 += kLanes) {
+        const float2 mine = i0 + lane < parts ? ml[(uint64_t)(i0 + lane) * BQ] : float2{-INFINITY, 0.0f};
+        const float w = mine.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mine.x - M);
+        L += w * mine.y;
+        const uint32_t n = min(parts - i0, kLanes);
+        for (uint32_t j0 = 0; j0 < n; j0 += 8) {
+            float4 a[8];
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j)  // past the last part: that part again, with no weight
+                a[j] = *reinterpret_cast<const float4 *>(po + (uint64_t)(i0 + min(j0 + j, n - 1)) * BQ * HD);
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) {
+                const float wj = j0 + j < n ? __shfl(w, (int)(j0 + j), (int)kLanes) : 0.0f;
+                o.x += wj * a[j].x;
+                o.y += wj * a[j].y;
+                o.z += wj * a[j].z;
+                o.w += wj * a[j].w;
+            }
+        }
+    }
+    L = pk::group_sum<kLanes>(L);
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    if (d >= p.Hd) return;  // padding dims of a kernel compiled for HD > Hd
+    typename O::storage *orow = out + ((uint64_t)bh * p.Sq + q) * p.Hd + d;
+    orow[0] = O::store(o.x * inv);
+    orow[1] = O::store(o.y * inv);
+    orow[2] = O::store(o.z * inv);
+    orow[3] = O::store(o.w * inv);
 }
 
 }  // namespace

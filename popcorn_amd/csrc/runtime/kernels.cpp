@@ -216,7 +216,10 @@ public:
             pairMergeInKernel_ = !(pm && std::string(pm) == "0");
             tiledName_ = std::string(rows16_ ? "flash_attention_tiled16_" : "flash_attention_tiled_") + tag(q.dataType) +
                          "_" + tag(out.dataType) + "_d" + std::to_string(hdp_);
+            mergeName_ = std::string("flash_attention_split_merge_") + tag(out_.dataType) + "_d" + std::to_string(hdp_);
             planTileSplit();
+            // the Hd 512 and f32 kernels run every tile whole
+            if (hdp_ != 512 && q_.dataType != DataType::f32) planRuns();
         }
         planSplit();
     }
@@ -228,7 +231,8 @@ public:
     }
 
     std::string describe() const override {
-        if (path_ == Kernels::AttentionPath::tiled) return nSplit_ && !mergedPairs() ? tiledName_ + "," + mergeName_ : tiledName_;
+        if (path_ == Kernels::AttentionPath::tiled)
+            return runLength_ || (nSplit_ && !mergedPairs()) ? tiledName_ + "," + mergeName_ : tiledName_;
         return partialName_ + "," + reduceName_;
     }
 
@@ -251,6 +255,7 @@ public:
             c.kvStride = (uint32_t)d_.cap;
             c.splitFrom = (uint32_t)(c.qTilesPerHead - nSplit_);
             c.pairTiles = pairTiles_ ? (mergedPairs() ? 2u : 1u) : 0u;
+            if (runLength_ && encodeRuns(enc, c)) return;
             // one block per tile; a split tile's two halves take two, a pair
             // of tiles two in all
             const int64_t items = d_.B * d_.Nq * ((int64_t)c.qTilesPerHead + (pairTiles_ ? 0 : nSplit_));
@@ -293,9 +298,8 @@ public:
                                       {q_, kRead}},
                                      {bytesOf(c)}, grid1(items, tiledBlock()));
                     enc.dispatch(fa);
-                    // one block per 16 rows of a split tile
                     FixedDispatch merge(mergeName_, {{pO, kRead}, {pML, kRead}, {out_, kWrite}}, {bytesOf(c)},
-                                        grid1(d_.B * d_.Nq * nSplit_ * 8, kBlock));
+                                        grid1(d_.B * d_.Nq * nSplit_ * mergeBlocksPerTile(), kBlock));
                     enc.dispatch(merge);
                 });
             });
@@ -309,6 +313,28 @@ public:
                     encodeSplit(enc, pO, pM, pL);
                 });
             });
+        });
+    }
+
+    // Runs of key steps: O, then (m, l), of every run's 128 rows in one scratch
+    // buffer. False, and nothing encoded, without it: the whole or paired
+    // tiles need none.
+    bool encodeRuns(KernelCommandEncoder &enc, TiledFlashAttentionConstants c) const {
+        const int64_t BH = d_.B * d_.Nq, rows = BH * runsPerHead_ * 128;
+        return enc.tryTemporaryTensor(ScratchSpec{{rows, hdp_ + 2}, DataType::f32}, [&](Tensor part) {
+            Tensor pO(part.data, Shape({rows, hdp_}), DataType::f32);
+            Tensor pML(static_cast<float *>(part.data) + rows * hdp_, Shape({rows, 2}), DataType::f32);
+            c.splitFrom = 0;
+            c.pairTiles = 3;
+            c.ticketLo = (uint32_t)runLength_;
+            c.ticketHi = (uint32_t)runsPerHead_;
+            FixedDispatch fa(tiledName_,
+                             {{q_, kRead}, {k_, kRead}, {v_, kRead}, {out_, kWrite}, {pO, kWrite}, {pML, kWrite}, {q_, kRead}},
+                             {bytesOf(c)}, grid1(BH * runsPerHead_, tiledBlock()));
+            enc.dispatch(fa);
+            FixedDispatch merge(mergeName_, {{pO, kRead}, {pML, kRead}, {out_, kWrite}}, {bytesOf(c)},
+                                grid1(BH * (int64_t)c.qTilesPerHead * mergeBlocksPerTile(), kBlock));
+            enc.dispatch(merge);
         });
     }
 
@@ -385,6 +411,59 @@ private:
     // and each pair runs as two blocks of equal work, when every pair splits
     // its heavy tile (x >= 1 steps in the first block); otherwise the tiles
     // with more than half the heaviest tile's steps run as two halves.
+    // Key steps of 32 that query tile qt of 128 rows visits (fa_steps).
+    int64_t keySteps(int64_t qt) const {
+        const int64_t first = d_.Sk - d_.Sq + qt * 128, last = d_.Sk - d_.Sq + std::min(qt * 128 + 127, d_.Sq - 1);
+        const int64_t hi = mask_.kind == 2 ? d_.Sk : std::min(d_.Sk, last + 1);
+        const int64_t lo = mask_.kind == 1 ? std::max<int64_t>(0, first - mask_.window + 1) : 0;
+        return hi > lo ? cdiv(hi - lo, 32) : 0;
+    }
+
+    // Runs (pairTiles 3): calls whose tiles leave CUs idle cut every tile's
+    // key steps into runs of at most L steps, one block each, merged by the
+    // merge kernel. L is the one of least estimated time,
+    //   rounds x L x t + 9 us + 8 us + 0.2 us per MB of partials,
+    // and runs are taken where that is under 0.9 of the whole or paired
+    // tiles' time, longest block x t + 9 us (+ 10 us for pairs' exchange),
+    // with t the time of a step (us, one block per CU; MI355X, fitted to L
+    // swept over 9 shapes per dtype). bf16, Hd 256, us before -> after: 500
+    // rows x 8692 keys, 8 heads 377 -> 68; 48 x 16000 684 -> 42; 1000 x 1000
+    // 43 -> 33; Hd 128, 300 x 3000, 32 heads 96 -> 46. Calls of under 768
+    // keys stay in one launch (a 640-key call's blocks run at most 12 steps
+    // as pairs).
+    void planRuns() {
+        const int64_t nQT = cdiv(d_.Sq, 128), BH = d_.B * d_.Nq, cus = deviceCUs();
+        if (d_.Sk < 768 || BH * nQT >= cus) return;
+        const bool bf = q_.dataType == DataType::bf16;
+        const double t = hdp_ == 256 ? (bf ? 1.37 : 1.04) : hdp_ == 128 ? (bf ? 0.90 : 0.71) : (bf ? 0.79 : 0.64);
+        std::vector<int64_t> n;
+        for (int64_t qt = 0; qt < nQT; ++qt) n.push_back(keySteps(qt));
+        const int64_t most = *std::max_element(n.begin(), n.end());
+        double best = (double)most * t + 9.0;
+        if (pairTiles_) {
+            double longest = 0.0;
+            for (int64_t i = 0; i < nQT / 2; ++i) longest = std::max(longest, 0.5 * (double)(n[i] + n[nQT - 1 - i]) + 1.0);
+            best = longest * t + 19.0;
+        }
+        best *= 0.9;
+        for (int64_t L = 1; L < most; ++L) {
+            int64_t items = 0, split = 0;
+            for (int64_t s : n) {
+                const int64_t runs = std::max<int64_t>(cdiv(s, L), 1);
+                items += runs;
+                split += runs > 1 ? runs : 0;
+            }
+            const double rounds = (double)cdiv(BH * items, cus);
+            if (rounds > 2.0) continue;
+            const double us = rounds * (double)L * t + 17.0 + 0.2 * 128.0 * 4e-6 * (double)(BH * split * hdp_);
+            if (us < best) {
+                best = us;
+                runLength_ = L;
+                runsPerHead_ = items;
+            }
+        }
+    }
+
     void planTileSplit() {
         nSplit_ = 0;
         pairTiles_ = false;
@@ -392,12 +471,7 @@ private:
         const int64_t tiles = d_.B * d_.Nq * nQT;
         // the Hd 512 and f32 kernels run every tile whole
         if (hdp_ == 512 || q_.dataType == DataType::f32 || mask_.kind != 0 || nQT < 4 || tiles > 2 * (int64_t)deviceCUs()) return;
-        auto steps = [&](int64_t qt) {
-            const int64_t last = d_.Sk - d_.Sq + std::min(qt * 128 + 127, d_.Sq - 1);
-            const int64_t hi = std::min(d_.Sk, last + 1);
-            return hi > 0 ? cdiv(hi, 32) : int64_t(0);
-        };
-        mergeName_ = std::string("flash_attention_split_merge_") + tag(out_.dataType) + "_d" + std::to_string(hdp_);
+        auto steps = [&](int64_t qt) { return keySteps(qt); };
         bool pairs = tiles <= (int64_t)deviceCUs();
         for (int64_t i = 0; pairs && i < nQT / 2; ++i) {
             const int64_t sa = steps(i), sb = steps(nQT - 1 - i);
@@ -439,11 +513,14 @@ private:
     int64_t partialBlock_ = kBlock;
     int64_t nSplit_ = 0;
     bool pairTiles_ = false;
+    int64_t runLength_ = 0, runsPerHead_ = 0;  // runs of key steps (0: none)
     bool rows16_ = false;  // the 16-rows-per-wave kernel: 8 waves per 128-row tile (4 per 64 at Hd 512 and in f32)
     int64_t hdp_ = 0;      // the tiled kernel's head dim: Hd padded to 64, 128, 256 or 512
     bool tiles64() const { return hdp_ == 512 || q_.dataType == DataType::f32; }
     int64_t tiledBlock() const { return tiles64() ? 256 : rows16_ ? 512 : kBlock; }
     int64_t tileRows() const { return tiles64() ? 64 : 128; }
+    // the merge kernel: HD / 4 lanes per row, so 1024 / HD of a tile's 128 rows per block
+    int64_t mergeBlocksPerTile() const { return 128 * hdp_ / 1024; }
     // Paired tiles are merged inside the tiled kernels (pairTiles 2).
     bool pairMergeInKernel_ = true;
     bool mergedPairs() const { return pairTiles_ && pairMergeInKernel_; }
