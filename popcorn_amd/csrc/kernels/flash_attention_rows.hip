@@ -1,0 +1,309 @@
+// FlashAttention for a few query rows (2 <= Sq < 32: a verified draft, the
+// tail of a chunked prompt) over f16 or bf16 K/V, on the matrix cores; the
+// reference's plain FlashAttention there (FlashAttention.swift:92-156).
+//
+// The G query heads of a KV head are packed into one set of R = Sq x G rows
+// (row r: query r / G, head r % G), so K and V are read once for all of them;
+// a block takes up to 16 RT of those rows. Its 4 waves take the 32-key steps
+// of the block's partition in turn, each with an online softmax of its own,
+// and merge in LDS. What bounds it is the latency of one pass over the cache
+// (8 heads, 4 KV heads, Hd 256, 8 rows x 4104 keys: 16.8 MB, 3.2 us at the
+// copy rate), so the steps are spread over as many waves as there are and
+// nothing is staged that a wave can load itself:
+//  * K fragments go global -> registers in the A layout of
+//    v_mfma_f32_16x16x32 (mfma.hpp): a lane's 16 bytes of one key row;
+//  * V goes global -> LDS by direct copies into the wave's own 32-key tile,
+//    row-major, and is read as the A operand of O^T += V^T . P^T by
+//    ds_read_b64_tr_b16: in each 16 lanes, lane i receives element i % 4 of
+//    the 8-byte pieces that lanes i / 4 + 4 j (j < 4) address, so lane s of
+//    group g, addressing key 4 g + s / 4 at dims 16 dt + 4 (s % 4), gets
+//    keys 4 g .. 4 g + 3 of dim 16 dt + s. Chunk c (16 bytes) of key row k
+//    sits in slot c ^ (2 (k % 8)) so the keys a read touches fall in
+//    different banks.
+// The one-row kernels (flash_decoding_partial_*) run per query row and read
+// K and V Sq times: 21.0 us for the call above, 11.7 here.
+//
+// Softmax: S^T = K . Q^T, so lane l holds the scores of row l % 16 for keys
+// 4 g + i and 16 + 4 g + i (g = l / 16), already the slots of its P^T
+// operand; maxima and sums run over lanes l, l ^ 16, l ^ 32. Weights enter
+// P.V in the input dtype, bf16 as a high part plus a remainder, and a row's
+// reference max moves only when a score passes it by more than 8 (natural
+// log), as in flash_attention_tiled.hip.
+#include <type_traits>
+
+#include "mfma.hpp"
+
+namespace {
+
+using pk::Mma16;
+using pk::u32x2;
+using pk::u32x4;
+
+constexpr int kWaves = 4;
+constexpr int BKV = 32;  // keys per step
+constexpr float kRescaleGap = 8.0f;
+constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+// past every head's range (the host keeps Sk * Hd * 2 below 2^31): zeros
+constexpr int kOutOfRange = (int)0x80000000u;
+
+typedef __attribute__((address_space(3))) void lds_void;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+__device__ inline float quad16_max(float v) { return pk::pair32_max(pk::pair16_max(v)); }
+__device__ inline float quad16_sum(float v) { return pk::pair32_sum(pk::pair16_sum(v)); }
+
+template <int N>
+__device__ inline void wait_vmcnt() {
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// pO [rows][P][Hd], pM, pL [rows][P] (rows as in q: b, head, query) for the
+// LSE combine (flash_decoding_reduce_*_ext; m in natural-log units), or with
+// P = 1 the output itself.
+template <typename T, typename O, int HD, int RT>
+__device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
+                        float *__restrict__ pO, float *__restrict__ pM, float *__restrict__ pL,
+                        typename O::storage *__restrict__ out, const FlashDecodingPartialExtConstants &p) {
+    constexpr int KS = HD / 32;                // k-steps of each S^T tile
+    constexpr int DT = HD / 16;                // 16-row tiles of O^T
+    constexpr int CH = HD / 8;                 // 16-byte chunks per row
+    constexpr int kRowsPer = 64 / CH;          // V rows per copy instruction
+    constexpr int kCopies = BKV / kRowsPer;    // copy instructions per step
+    constexpr int kVary = 8 / kRowsPer;        // distinct chunk swizzles over the instructions
+    constexpr bool kSplitP = std::is_same<T, pk::BF16>::value;
+    constexpr int LDO = HD + 4;                // merged-state row, in floats
+    static_assert(CH <= 64 && kVary >= 1, "a V row is at most one instruction, at least 8 to a swizzle period");
+    constexpr int kStage = kWaves * BKV * HD * 2, kMerge = kWaves * 16 * LDO * 4;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[kStage > kMerge ? kStage : kMerge];
+    __shared__ float sm_m[kWaves][RT * 16], sm_l[kWaves][RT * 16];
+
+    const uint32_t lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t D = p.Hd, G = p.Nq / p.Nkv, R = p.Sq * G, P = p.P;
+    const uint32_t groups = (R + 16 * RT - 1) / (16 * RT);
+    const uint32_t bkv = blockIdx.y / groups, r0 = blockIdx.y % groups * (16 * RT);
+    const uint32_t b = bkv / p.Nkv, hkv = bkv % p.Nkv;
+    const uint64_t kvoff = (uint64_t)bkv * (p.kvStride ? p.kvStride : p.Sk) * D;
+    auto q_row = [&](uint32_t r) { return ((uint64_t)b * p.Nq + hkv * G + r % G) * p.Sq + r / G; };
+
+    // rows past R repeat the last one and are not stored
+    u32x4 qf[RT][KS];
+    int posQ[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const uint32_t r = min(r0 + rt * 16 + c16, R - 1);
+        posQ[rt] = (int)p.Sk - (int)p.Sq + (int)(r / G);
+        const uint16_t *row = Q + q_row(r) * D + g * 8;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            qf[rt][s] = s * 32 + g * 8 < D ? *reinterpret_cast<const u32x4 *>(row + s * 32) : u32x4{0u, 0u, 0u, 0u};
+    }
+
+    // keys that some row of the block sees, in steps; this partition's steps
+    const int first = (int)p.Sk - (int)p.Sq + (int)(r0 / G);
+    const int last = (int)p.Sk - (int)p.Sq + (int)(min(r0 + 16 * RT, R) - 1) / (int)G;
+    const int kLo = p.maskKind == 1u ? max(0, first - p.slidingWindow + 1) : 0;
+    const int kHi = p.maskKind == 2u ? (int)p.Sk : min((int)p.Sk, last + 1);
+    const uint32_t n = kHi > kLo ? (uint32_t)(kHi - kLo + BKV - 1) / BKV : 0u;
+    const uint32_t hi = (uint32_t)((uint64_t)n * (blockIdx.x + 1) / P);
+    uint32_t it = (uint32_t)((uint64_t)n * blockIdx.x / P) + wave;
+
+    const __amdgpu_buffer_rsrc_t rsK = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(K + kvoff), 0,
+                                                                          (int)(p.Sk * D * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsV = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(V + kvoff), 0,
+                                                                          (int)(p.Sk * D * 2), 0x00020000);
+    u32x4 kf[2][KS];
+    // a step past the partition reads out of range: zeros, no memory read
+    auto loadK = [&](uint32_t step) {
+        const int so = step < hi ? (int)((uint32_t)(kLo + (int)step * BKV) * D * 2) : kOutOfRange;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const uint32_t d = s * 32 + g * 8;
+                const int off = d < D ? (int)(((mt * 16 + c16) * D + d) * 2) : kOutOfRange;
+                kf[mt][s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsK, off, so, 0));
+            }
+    };
+    // V copies: instruction i writes rows i kRowsPer .. of the wave's tile
+    uint8_t *sV = smem + wave * (BKV * HD * 2);
+    int voff[kVary];
+#pragma unroll
+    for (int i = 0; i < kVary; ++i) {
+        const uint32_t row = lane / CH, key = i * kRowsPer + row, chunk = (lane % CH) ^ (2 * (key % 8) % CH);
+        voff[i] = chunk * 8 < D ? (int)((row * D + chunk * 8) * 2) : kOutOfRange;
+    }
+    auto copyV = [&](uint32_t step) {
+        const int so = (int)((uint32_t)(kLo + (int)step * BKV) * D * 2);
+#pragma unroll
+        for (int i = 0; i < kCopies; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsV, (lds_void *)(sV + i * 1024), 16, voff[i % kVary],
+                                                     so + (int)(i * kRowsPer * D * 2), 0, 0);
+    };
+    // this lane's 8-byte piece of key row `key` at dim tile dt
+    auto readV = [&](int dt, uint32_t key) {
+        const uint32_t chunk = (2 * dt + (c16 & 3) / 2) ^ (2 * (key % 8) % CH);
+        const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(sV + key * (HD * 2) + chunk * 16 + (c16 & 1) * 8));
+        return __builtin_bit_cast(u32x2, v);
+    };
+
+    const float c2 = p.scale * kLog2e;
+    pk::f32x4 acc[RT][DT];
+    float m[RT], l[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        m[rt] = -INFINITY;
+        l[rt] = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[rt][dt] = pk::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    loadK(it);
+    for (; it < hi; it += kWaves) {
+        const int k0 = kLo + (int)it * BKV;
+        copyV(it);
+        pk::f32x4 st[RT][2];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) {
+                st[rt][mt] = pk::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int s = 0; s < KS; ++s) st[rt][mt] = Mma16<T>::run(kf[mt][s], qf[rt][s], st[rt][mt]);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        loadK(it + kWaves);
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 pf[RT], pfr[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            float sv[8], mx = -INFINITY, ps = 0.0f, alpha = 1.0f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int key = k0 + (i / 4) * 16 + (int)g * 4 + i % 4;
+                const bool ok = (key < (int)p.Sk) & ((p.maskKind == 2u) | (key <= posQ[rt])) &
+                                ((p.maskKind != 1u) | (posQ[rt] - key < p.slidingWindow));
+                sv[i] = ok ? st[rt][i / 4][i % 4] : -INFINITY;
+                mx = fmaxf(mx, sv[i]);
+            }
+            mx = quad16_max(mx) * c2;
+            const bool move = mx > m[rt] + kRescaleGap * kLog2e;
+            if (move) {
+                alpha = __builtin_amdgcn_exp2f(m[rt] - mx);
+                m[rt] = mx;
+            }
+            if (__ballot(move)) {
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) acc[rt][dt] *= alpha;
+            }
+            // a row that has seen no key yet: every weight 0
+            const float mref = m[rt] == -INFINITY ? 0.0f : m[rt];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(sv[2 * j], c2, -mref));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(sv[2 * j + 1], c2, -mref));
+                ps += p0 + p1;
+                const uint32_t w = pk::pack2<T>(p0, p1);
+                pf[rt][j] = w;
+                if constexpr (kSplitP)
+                    pfr[rt][j] = pk::pack2<T>(p0 - __uint_as_float(w << 16), p1 - __uint_as_float(w & 0xffff0000u));
+            }
+            l[rt] = l[rt] * alpha + quad16_sum(ps);
+        }
+        wait_vmcnt<2 * KS>();  // the V copies; the next step's K loads stay in flight
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            const u32x2 lo = readV(dt, 4 * g + c16 / 4), hi2 = readV(dt, 16 + 4 * g + c16 / 4);
+            const u32x4 va = {lo.x, lo.y, hi2.x, hi2.y};
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                acc[rt][dt] = Mma16<T>::run(va, pf[rt], acc[rt][dt]);
+                if constexpr (kSplitP) acc[rt][dt] = Mma16<T>::run(va, pfr[rt], acc[rt][dt]);
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // this wave's reads of its V tile are done before it is overwritten
+        asm volatile("" ::: "memory");
+    }
+    wait_vmcnt<0>();  // the last K loads (zeros), before their registers go
+
+    // merge the waves' states, one tile of 16 rows at a time: O through LDS,
+    // thread t takes row t / 16, dims 4 (t % 16) + 64 j
+    if (g == 0) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            sm_m[wave][rt * 16 + c16] = m[rt];
+            sm_l[wave][rt * 16 + c16] = l[rt];
+        }
+    }
+    float *sO = reinterpret_cast<float *>(smem);
+    const uint32_t tr = threadIdx.x / 16, td = threadIdx.x % 16 * 4;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        __syncthreads();  // V tiles and the previous tile's state are read
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+            *reinterpret_cast<pk::f32x4 *>(&sO[(wave * 16 + c16) * LDO + dt * 16 + g * 4]) = acc[rt][dt];
+        __syncthreads();
+        const uint32_t r = r0 + rt * 16 + tr;
+        if (r >= R) continue;
+        float M = -INFINITY, w[kWaves], L = 0.0f;
+#pragma unroll
+        for (int v = 0; v < kWaves; ++v) M = fmaxf(M, sm_m[v][rt * 16 + tr]);
+#pragma unroll
+        for (int v = 0; v < kWaves; ++v) {
+            const float mv = sm_m[v][rt * 16 + tr];
+            w[v] = mv == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mv - M);
+            L += w[v] * sm_l[v][rt * 16 + tr];
+        }
+        const uint64_t slot = q_row(r) * P + blockIdx.x;
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        for (uint32_t d = td; d < D; d += 64) {
+            pk::f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int v = 0; v < kWaves; ++v) o += *reinterpret_cast<const pk::f32x4 *>(&sO[(v * 16 + tr) * LDO + d]) * w[v];
+            if (P > 1) {
+                *reinterpret_cast<pk::f32x4 *>(pO + slot * D + d) = o;
+            } else {
+                typename O::storage *dst = out + slot * D + d;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dst[i] = O::store(o[i] * inv);
+            }
+        }
+        if (P > 1 && td == 0) {
+            pM[slot] = M * kLn2;
+            pL[slot] = L;
+        }
+    }
+}
+
+}  // namespace
+
+// Two blocks per CU where a wave fits 256 registers.
+#define FA_ROWS(name, T, O, HD, RT, PER_CU)                                                                      \
+    POPCORN_KERNEL void __launch_bounds__(256, PER_CU)                                                           \
+        name(const uint16_t *q, const uint16_t *k, const uint16_t *v, float *pO, float *pM, float *pL,           \
+             O::storage *out, FlashDecodingPartialExtConstants p) {                                              \
+        fa_rows<T, O, HD, RT>(q, k, v, pO, pM, pL, out, p);                                                      \
+    }
+#define FA_ROWS_D(t, T, o, O)                                                       \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d64_r1, T, O, 64, 1, 2)                \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d64_r2, T, O, 64, 2, 2)                \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d64_r4, T, O, 64, 4, 2)                \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d128_r1, T, O, 128, 1, 2)              \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d128_r2, T, O, 128, 2, 2)              \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d128_r4, T, O, 128, 4, 1)              \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d256_r1, T, O, 256, 1, 2)              \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d256_r2, T, O, 256, 2, 1)              \
+    FA_ROWS(flash_attention_rows_##t##_##o##_d512_r1, T, O, 512, 1, 1)
+
+using pk::BF16;
+using pk::F16;
+using pk::F32;
+
+FA_ROWS_D(f16, F16, f16, F16)
+FA_ROWS_D(f16, F16, f32, F32)
+FA_ROWS_D(bf16, BF16, bf16, BF16)
+FA_ROWS_D(bf16, BF16, f32, F32)

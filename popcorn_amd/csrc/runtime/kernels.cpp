@@ -222,6 +222,7 @@ public:
             if (hdp_ != 512 && q_.dataType != DataType::f32) planRuns();
         }
         planSplit();
+        planRows();
     }
 
     std::vector<Binding> tensors() const override {
@@ -233,10 +234,15 @@ public:
     std::string describe() const override {
         if (path_ == Kernels::AttentionPath::tiled)
             return runLength_ || (nSplit_ && !mergedPairs()) ? tiledName_ + "," + mergeName_ : tiledName_;
+        if (rowTiles_) return rowsP_ > 1 ? rowsName_ + "," + reduceName_ : rowsName_;
         return partialName_ + "," + reduceName_;
     }
 
     void encode(KernelCommandEncoder &enc) const override {
+        if (rowTiles_) {
+            encodeRows(enc);
+            return;
+        }
         if (path_ == Kernels::AttentionPath::tiled) {
             // TiledFlashAttentionConstants (the fields of
             // PopcornKernelTypes.h:133-144 and two more): one block per 128
@@ -360,22 +366,13 @@ public:
 
     // Forces the split-KV kernels (the plain/decoding routes) whatever route
     // the shape would take.
-    void useSplitPath() { path_ = Kernels::AttentionPath::decoding; }
+    void useSplitPath() {
+        path_ = Kernels::AttentionPath::decoding;
+        rowTiles_ = 0;
+    }
 
     void encodeSplit(KernelCommandEncoder &enc, const Tensor &pO, const Tensor &pM, const Tensor &pL) const {
-        FlashDecodingPartialExtConstants pc{};
-        pc.B = (uint32_t)d_.B;
-        pc.Nq = (uint32_t)d_.Nq;
-        pc.Nkv = (uint32_t)d_.Nkv;
-        pc.Sk = (uint32_t)d_.Sk;
-        pc.Hd = (uint32_t)d_.Hd;
-        pc.P = (uint32_t)P_;
-        pc.maskKind = mask_.kind;
-        pc.slidingWindow = mask_.kind == 1 ? mask_.window : -1;
-        pc.scale = scale_;
-        pc.kvStride = (uint32_t)d_.cap;
-        pc.Sq = (uint32_t)d_.Sq;
-        pc.keyLenFromPosition = hasPos_ ? 1u : 0u;
+        FlashDecodingPartialExtConstants pc = partialConstants(P_);
         DispatchSize ds;
         ds.grid = dim3((unsigned)P_, (unsigned)(d_.B * d_.Nkv * ngroups_), (unsigned)d_.Sq);
         ds.block = dim3((unsigned)partialBlock_, 1, 1);
@@ -386,11 +383,59 @@ public:
                                {posOrDummy, kRead}},
                               {bytesOf(pc)}, ds);
         enc.dispatch(partial);
+        encodeReduce(enc, pO, pM, pL, P_);
+    }
+
+    // A few query rows on the matrix cores: the partial states of rowsP_
+    // partitions and their combine, or without scratch for them one partition.
+    void encodeRows(KernelCommandEncoder &enc) const {
+        const int64_t rows = d_.B * d_.Nq * d_.Sq, slots = rows * rowsP_;
+        auto launch = [&](int64_t P, const Tensor &pO, const Tensor &pM, const Tensor &pL) {
+            DispatchSize ds;
+            ds.grid = dim3((unsigned)P, (unsigned)(d_.B * d_.Nkv * cdiv(d_.Sq * (d_.Nq / d_.Nkv), 16 * rowTiles_)), 1);
+            ds.block = dim3(kBlock, 1, 1);
+            // with one partition the output is written and the partials are not; else the other way round
+            FixedDispatch fa(rowsName_,
+                             {{q_, kRead}, {k_, kRead}, {v_, kRead}, {pO, P > 1 ? kWrite : kRead},
+                              {pM, P > 1 ? kWrite : kRead}, {pL, P > 1 ? kWrite : kRead}, {out_, kWrite}},
+                             {bytesOf(partialConstants(P))}, ds);
+            enc.dispatch(fa);
+        };
+        if (rowsP_ > 1 && enc.tryTemporaryTensor(ScratchSpec{{slots, d_.Hd + 2}, DataType::f32}, [&](Tensor part) {
+                float *base = static_cast<float *>(part.data);
+                Tensor pO(base, Shape({slots, d_.Hd}), DataType::f32);
+                Tensor pM(base + slots * d_.Hd, Shape({slots}), DataType::f32);
+                Tensor pL(base + slots * (d_.Hd + 1), Shape({slots}), DataType::f32);
+                launch(rowsP_, pO, pM, pL);
+                encodeReduce(enc, pO, pM, pL, rowsP_);
+            }))
+            return;
+        launch(1, q_, q_, q_);
+    }
+
+    FlashDecodingPartialExtConstants partialConstants(int64_t P) const {
+        FlashDecodingPartialExtConstants pc{};
+        pc.B = (uint32_t)d_.B;
+        pc.Nq = (uint32_t)d_.Nq;
+        pc.Nkv = (uint32_t)d_.Nkv;
+        pc.Sk = (uint32_t)d_.Sk;
+        pc.Hd = (uint32_t)d_.Hd;
+        pc.P = (uint32_t)P;
+        pc.maskKind = mask_.kind;
+        pc.slidingWindow = mask_.kind == 1 ? mask_.window : -1;
+        pc.scale = scale_;
+        pc.kvStride = (uint32_t)d_.cap;
+        pc.Sq = (uint32_t)d_.Sq;
+        pc.keyLenFromPosition = hasPos_ ? 1u : 0u;
+        return pc;
+    }
+
+    void encodeReduce(KernelCommandEncoder &enc, const Tensor &pO, const Tensor &pM, const Tensor &pL, int64_t P) const {
         FlashDecodingReduceExtConstants rc{};
         rc.B = (uint32_t)d_.B;
         rc.Nq = (uint32_t)d_.Nq;
         rc.Hd = (uint32_t)d_.Hd;
-        rc.P = (uint32_t)P_;
+        rc.P = (uint32_t)P;
         rc.Sq = (uint32_t)d_.Sq;
         // one block per (query row, 64-dim slice of the head)
         DispatchSize rs;
@@ -417,6 +462,36 @@ private:
         const int64_t hi = mask_.kind == 2 ? d_.Sk : std::min(d_.Sk, last + 1);
         const int64_t lo = mask_.kind == 1 ? std::max<int64_t>(0, first - mask_.window + 1) : 0;
         return hi > lo ? cdiv(hi - lo, 32) : 0;
+    }
+
+    // 2 to 31 query rows over 16-bit K/V in 16-byte rows: flash_attention_rows_*
+    // (flash_attention_rows.hip), which reads K and V once for all the rows
+    // of a KV head's query heads. Row tiles of 16 per block: as many as the
+    // kernels have and the rows half fill, where blocks of 8 key steps (two
+    // per wave) still fill the CUs, since then K/V traffic counts (4
+    // sequences, 32 / 8 heads, Hd 128, 16 rows x 8000 keys: 4 tiles 52 us, 1
+    // tile 64); else one (31 rows x 2000 keys, 8 heads on one, Hd 256: 1 tile
+    // 15.3 us, 2 tiles 18.4). Partitions: one block per CU, a step per wave at
+    // least (8 rows x 4104 keys, 4 KV heads: 33 partitions 12.2 us, 17 14.1,
+    // 65 13.7); up to 12 steps one partition, which needs no combine (100
+    // keys: 4.2 against 7.6 us). Before, per row: 507, 62.4 and 22.7 us.
+    void planRows() {
+        const int64_t lim = int64_t{1} << 31, G = d_.Nq / d_.Nkv, R = d_.Sq * G, cus = deviceCUs();
+        const DataType t = q_.dataType;
+        if (d_.Sq < 2 || d_.Sq >= 32 || hasPos_ || !(t == DataType::f16 || t == DataType::bf16) || d_.Hd % 8 != 0 ||
+            !(out_.dataType == t || out_.dataType == DataType::f32) || !aligned16(q_.data) || !aligned16(k_.data) ||
+            !aligned16(v_.data) || !(scale_ > 0.0f) || d_.Sk <= 0 || d_.Sk * d_.Hd * 2 >= lim ||
+            d_.B * d_.Nkv * cdiv(R, 16) > 65535)
+            return;
+        const int64_t hdp = d_.Hd <= 64 ? 64 : d_.Hd <= 128 ? 128 : d_.Hd <= 256 ? 256 : 512;
+        const int64_t keys = mask_.kind == 1 ? std::min<int64_t>(d_.Sk, std::max<int64_t>(mask_.window, 0) + d_.Sq) : d_.Sk;
+        const int64_t steps = cdiv(keys, 32);
+        auto blocks = [&](int64_t rt) { return d_.B * d_.Nkv * cdiv(R, 16 * rt); };
+        rowTiles_ = hdp <= 128 ? 4 : hdp == 256 ? 2 : 1;
+        while (rowTiles_ > 1 && (R <= 8 * rowTiles_ || blocks(rowTiles_) * cdiv(steps, 8) < cus)) rowTiles_ /= 2;
+        rowsP_ = steps <= 12 ? 1 : std::clamp<int64_t>(cus / blocks(rowTiles_), 1, cdiv(steps, 4));
+        rowsName_ = std::string("flash_attention_rows_") + tag(t) + "_" + tag(out_.dataType) + "_d" + std::to_string(hdp) +
+                    "_r" + std::to_string(rowTiles_);
     }
 
     // Runs (pairTiles 3): calls whose tiles leave CUs idle cut every tile's
@@ -514,6 +589,8 @@ private:
     int64_t nSplit_ = 0;
     bool pairTiles_ = false;
     int64_t runLength_ = 0, runsPerHead_ = 0;  // runs of key steps (0: none)
+    int64_t rowTiles_ = 0, rowsP_ = 1;         // a few rows on the matrix cores (0: not)
+    std::string rowsName_;
     bool rows16_ = false;  // the 16-rows-per-wave kernel: 8 waves per 128-row tile (4 per 64 at Hd 512 and in f32)
     int64_t hdp_ = 0;      // the tiled kernel's head dim: Hd padded to 64, 128, 256 or 512
     bool tiles64() const { return hdp_ == 512 || q_.dataType == DataType::f32; }

@@ -1,0 +1,108 @@
+"""Attention of 2 to 31 query rows on the matrix cores (flash_attention_rows_*):
+the rule that takes a call there on the CPU, outputs against the oracle on the
+GPU at the edges of row tiles, key steps, partitions and head dims."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+
+FAKE = 1 << 20
+
+
+def _kernel(pa, t, B, Nq, Nkv, Sq, Sk, cap, Hd, mask=(0, -1), scale=None, q=None, k=None, v=None, out=None, ot=None, **kw):
+    def fake(*shape):
+        return pa.Tensor(FAKE, shape, t)
+
+    q, out = q or fake(B, Nq, Sq, Hd), out or pa.Tensor(FAKE, (B, Nq, Sq, Hd), ot or t)
+    k, v = k or fake(B, Nkv, cap, Hd), v or fake(B, Nkv, cap, Hd)
+    return pa.Kernels.FlashAttention(q, k, v, out=out, scale=Hd ** -0.5 if scale is None else scale,
+                                     mask=pa.AttentionMask(*mask), batch=B, query_heads=Nq, kv_heads=Nkv, query_len=Sq,
+                                     key_len=Sk, head_dim=Hd, key_capacity=cap, **kw)
+
+
+def test_rows_rule():
+    import popcorn_amd as pa
+
+    def name(Nq, Nkv, Sq, Sk, Hd=256, t="bf16", **kw):
+        return _kernel(pa, t, 1, Nq, Nkv, Sq, Sk, Sk, Hd, **kw).function_names
+
+    assert name(8, 4, 8, 4104) == ["flash_attention_rows_bf16_bf16_d256_r1", "flash_decoding_reduce_bf16_ext"]
+    assert name(8, 4, 8, 384) == ["flash_attention_rows_bf16_bf16_d256_r1"]  # 12 steps: one partition
+    assert name(32, 8, 31, 30000, 128)[0] == "flash_attention_rows_bf16_bf16_d128_r4"
+    assert name(8, 8, 2, 200, 72, ot="f32") == ["flash_attention_rows_bf16_f32_d128_r1"]
+    old = "flash_decoding_partial_"
+    assert name(8, 4, 1, 4104)[0].startswith(old)
+    assert name(8, 4, 8, 4104, t="f32")[0].startswith(old)
+    assert name(8, 4, 8, 4104, 252)[0].startswith(old)        # rows not in 16-byte chunks
+    assert name(8, 4, 8, 4104, scale=-1.0)[0].startswith(old)  # maxima are taken on unscaled scores
+    pos = pa.Tensor(FAKE, (1,), "i32")
+    assert name(8, 4, 8, 4104, position=pos)[0].startswith(old)
+    q = pa.Tensor(FAKE + 2, (1, 8, 8, 256), "bf16")
+    assert name(8, 4, 8, 4104, q=q)[0].startswith(old)
+    assert name(8, 4, 8, 4104, ot="f16")[0].startswith(old)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t,ot", [("f16", "f16"), ("bf16", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("B,Nq,Nkv,Sq,Sk,cap,Hd,mask", [
+    (1, 2, 2, 2, 2, 2, 64, (0, -1)),            # fewer keys than a step, rows of one head
+    (1, 4, 2, 8, 33, 40, 256, (0, -1)),         # 16 rows exactly; a second step of one key
+    (2, 6, 2, 11, 500, 512, 128, (0, -1)),      # 33 rows: a third tile of one row; 16 steps: partitions
+    (1, 8, 1, 31, 1100, 1100, 256, (0, -1)),    # 248 rows of one KV head
+    (1, 2, 1, 5, 700, 701, 512, (0, -1)),
+    (1, 4, 4, 3, 450, 450, 200, (2, -1)),       # padded head dim, every key
+    (1, 4, 2, 9, 900, 1000, 72, (1, 100)),      # a window: most partitions of the keys unseen
+    (1, 4, 1, 20, 600, 600, 128, (1, 3)),
+    (8, 32, 8, 16, 2050, 2050, 64, (0, -1)),    # 4 row tiles per block
+    (8, 16, 8, 16, 1100, 1100, 256, (0, -1)),   # 2 row tiles per block
+])
+def test_rows_vs_oracle(t, ot, B, Nq, Nkv, Sq, Sk, cap, Hd, mask):
+    import oracle as O
+    from conftest import assert_out
+    from gpu_util import EPS, download, gpu_env, rounded, upload
+
+    pa, lib, stream, enc = gpu_env()
+    q = rounded(O.normal(Sq, (B, Nq, Sq, Hd)), t)
+    k, v = (rounded(O.normal(Sk + i, (B, Nkv, cap, Hd)), t) for i in (1, 2))
+    k[:, :, Sk:] = v[:, :, Sk:] = np.nan  # rows past the keys
+    guard = 64
+    buf = upload(pa, np.full(q.size + guard, 7.0, np.float32), ot)
+    kern = _kernel(pa, t, B, Nq, Nkv, Sq, Sk, cap, Hd, mask, None, upload(pa, q, t), upload(pa, k, t), upload(pa, v, t),
+                   buf.view([B, Nq, Sq, Hd]))
+    assert kern.function_names[0].startswith("flash_attention_rows_")
+    ref = O.attention_naive(q, k, v, Hd ** -0.5, key_len=Sk, mask_kind=mask[0], window=mask[1])
+
+    class Empty(pa.KernelScratchAllocator):
+        def borrow(self, length):
+            raise MemoryError
+
+    # with the plan's partitions, and with no scratch for them: one partition
+    for e in (enc, pa.KernelCommandEncoder(lib, stream, Empty())):
+        buf.copy_from(np.full(q.size + guard, 7.0, np.float32) if ot == "f32" else
+                      O.to_bits(np.full(q.size + guard, 7.0, np.float32), {"f16": O.F16, "bf16": O.BF16}[ot]), stream)
+        e.encode(kern)
+        stream.synchronize()
+        got = download(buf, stream)
+        assert (got[q.size:] == 7.0).all(), "wrote past the output"
+        assert_out(got[:q.size].reshape(q.shape), ref, EPS[t], ot, f"rows {kern.function_names}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", ["f16", "bf16"])
+def test_rows_wide_score_range(t):
+    # scores over hundreds of natural-log units: the reference max moves on
+    # most steps, in waves and partitions of their own
+    import oracle as O
+    from conftest import assert_out
+    from gpu_util import EPS, download, gpu_env, rounded, upload
+
+    pa, lib, stream, enc = gpu_env()
+    q, k = (rounded(3.0 * O.normal(s, sh), t) for s, sh in ((1, (1, 4, 7, 256)), (2, (1, 2, 640, 256))))
+    v = rounded(O.normal(3, (1, 2, 640, 256)), t)
+    out = pa.Tensor.empty([1, 4, 7, 256], t)
+    enc.encode(_kernel(pa, t, 1, 4, 2, 7, 640, 640, 256, (0, -1), 1.0, upload(pa, q, t), upload(pa, k, t), upload(pa, v, t), out))
+    stream.synchronize()
+    assert_out(download(out, stream), O.attention_naive(q, k, v, 1.0), EPS[t], t, "wide range")
