@@ -2101,6 +2101,45 @@ private:
     AffineQMatmulConstants qc_;
 };
 
+// A few bf16 rows through a 4-bit matrix (aq_rows.hip): the row tiles of 16,
+// the waves that share a tile's K, and the values of K staged per phase.
+struct AqRowsPlan {
+    int mt = 0, wk = 1;  // mt 0: not this kernel
+    int64_t kp = 0;
+    size_t lds = 0;
+};
+
+AqRowsPlan aqRowsPlan(int64_t m, int64_t n, int64_t k) {
+    AqRowsPlan r;
+    // Against one matvec per row (m < 16, or under 2^27 weight bytes in all),
+    // whose time grows with m n k while this kernel's fixed cost is 5-6 us:
+    // from 25 million multiply-adds on (K 2304, N 2304: m 4 6.2 against 6.3 us,
+    // m 8 8.4 against 6.5), two rows from 2^26 (K 2304, N 9216: 9.1 against
+    // 9.9; K 3072, N 24576: 20.6 against 17.7), and not below 1024 rows of W
+    // (K 8192, N 500, m 8: 8.1 against 11.5).
+    if (m < 2 || m > 64 || n < 1024 || m * n * k < (m == 2 ? int64_t{1} << 26 : 25000000)) return r;
+    // Against the prompt GEMM (aq_gemm.hip): up to 48 rows, while x fits one or
+    // two phases (K 2304, N 9216, m 16: 22.1 against 10.9 us, m 48 27.1 against
+    // 22.8; K 9216, N 2304, m 24 28.8 against 23.8, m 32 29.8 against 30.9).
+    // K under 2048 stays there too: the routing tests hold it (K 1024, N 16448,
+    // m 16: 19.5 against 7.6).
+    if (m >= kQ4GemmMinRows && m * n * (k / 2) >= kQ4GemmMinBytes && (k < 2048 || m > 48)) return r;
+    if (m >= kQ4GemmMinRows && m * k > (m <= 32 ? 230000 : 165000)) return r;
+    r.mt = m <= 16 ? 1 : m <= 32 ? 2 : 4;
+    // the fewest waves per tile (x is staged once per block) that give more
+    // blocks than half the CUs: N 9216 144 blocks of 4 tiles (288 of 2 tiles:
+    // 11.3 us), N 4096 256 blocks of one (128 of two: 8.1 against 7.0)
+    while (r.wk < 8 && cdiv(n, 16 * (8 / r.wk)) * 2 <= deviceCUs()) r.wk *= 2;
+    // x and its group sums in up to 152 KB of LDS, in equal phases
+    auto bytes = [&](int64_t kp) { return (size_t)(m * (kp * 2 + 16) + kp / 64 * 16 * r.mt * 4); };
+    for (int64_t phases = 1;; ++phases) {
+        r.kp = cdiv(k / 128, phases) * 128;
+        if (bytes(r.kp) <= 152 * 1024 || r.kp == 128) break;
+    }
+    r.lds = std::max(bytes(r.kp), (size_t)(8 * r.mt * 1024));  // the waves' sums take its place at the end
+    return r;
+}
+
 // Matmul.swift:99-130 and :279-332
 std::unique_ptr<Kernel> Matmul(const Tensor &a, const AffineQuantizedTensor &b, const Tensor &c) {
     using D = DataType;
@@ -2137,12 +2176,21 @@ std::unique_ptr<Kernel> Matmul(const Tensor &a, const AffineQuantizedTensor &b, 
     const Q4Shape q = q4Shape(n, k, x == D::f32);
     const bool aligned = aligned16(b.packedValues.data) && aligned16(a.data) &&
                          (reinterpret_cast<uintptr_t>(b.scales.data) & 3) == 0 && (reinterpret_cast<uintptr_t>(bias.data) & 3) == 0;
+    const int64_t lim = int64_t{1} << 31;
+    if (x == D::bf16 && o == D::bf16 && aligned && k % 128 == 0 && n * (k / 2) < lim && m * k * 2 < lim) {
+        const AqRowsPlan r = aqRowsPlan(m, n, k);
+        if (r.mt) {
+            const uint32_t kp = (uint32_t)r.kp;
+            return std::make_unique<FixedDispatch>(
+                "aq_matvec_simd4_" + combo3 + "_m" + std::to_string(r.mt) + "_s" + std::to_string(r.wk), binds,
+                std::vector<std::vector<uint8_t>>{bytesOf(qc), bytesOf(kp)}, grid1(cdiv(n, 16 * (8 / r.wk)), 512, r.lds));
+        }
+    }
     // a prompt's rows of bf16 activations: the matrix-core GEMM (one pass
     // over the weights for all rows instead of one matvec per row)
     // (buffer copies: every operand under 2^31 bytes; an even number of
     // groups per row, so a group's scale and bias share a 32-bit word with
     // a neighbour of the same row)
-    const int64_t lim = int64_t{1} << 31;
     if (x == D::bf16 && m >= kQ4GemmMinRows && m * n * (k / 2) >= kQ4GemmMinBytes && aligned && k % 128 == 0 &&
         m * k * 2 < lim && n * (k / 2) < lim && m * (k / 64) * 4 < lim && cdiv(m, 128) * cdiv(n, 128) <= (int64_t)UINT32_MAX)
         return std::make_unique<AffineQGemmKernel>(a, b, c, qc);
