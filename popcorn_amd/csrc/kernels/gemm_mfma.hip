@@ -488,7 +488,11 @@ __device__ void gemm_splitk_reduce(const float *__restrict__ P, typename O::stor
     }
 #define GEMM_MFMA_TILES(base, T, O)                          \
     GEMM_MFMA_E(base##_e256x384, T, O, 256, 384, 2, 4)       \
+    GEMM_MFMA_E(base##_e256x320, T, O, 256, 320, 4, 2)       \
+    GEMM_MFMA_E(base##_e192x384, T, O, 192, 384, 3, 4)       \
     GEMM_MFMA_E(base##_e256x288, T, O, 256, 288, 4, 3)       \
+    GEMM_MFMA_E(base##_e256x192, T, O, 256, 192, 4, 2)       \
+    GEMM_MFMA_E(base##_e192x256, T, O, 192, 256, 3, 4)       \
     GEMM_MFMA_E(base##_e256x256, T, O, 256, 256, 2, 4)       \
     GEMM_MFMA_E(base##_e128x128, T, O, 128, 128, 2, 2)       \
     GEMM_MFMA_E(base##_e128x256, T, O, 128, 256, 2, 4)       \

@@ -856,34 +856,45 @@ bool gemmLinesFit(int64_t k, int bn) { return k % 64 != 32 && gemmOffsetsFit(k, 
 // their grid keeps busy over its rounds (two blocks per CU for the tiles
 // of at most 80 KB of LDS; such a tile alone on a CU counts 0.6 of a
 // slot), times the share of the grid's tiles that lies inside C, times the
-// tile's measured throughput per CU relative to 256 x 384 when the CUs are
-// full (bf16, 33 Gemma-family prefill shapes, M 512-4096: the score's pick
-// was within 3% of the fastest tile on 31 and within 5% on the others,
-// 5% faster than the rules of the 64-byte-row tiles over all of them).
+// tile's throughput per CU relative to 256 x 384 when the CUs are full.
+// A first round that gives only some CUs their second block is paid in full
+// by those: 0.78, measured at M > 512 and K <= 4096 (M 1000, K 2304, N 9216,
+// 384 tiles of 128 x 192: 53.4 us, 192 of 256 x 192: 45.0); with fewer rows
+// or longer K the larger tiles gave nothing (M 594, K 9216, N 14336: 187
+// and 197).
+// The weights are fitted to every tile's time on 131 shapes (bf16, M 65-4700,
+// K 1024-14336, N 2304-256000, more than two 128 x 128 tiles per CU): the
+// score's pick is on average 0.6% slower than the fastest tile (the six tiles
+// before 192 x 384, 192 x 256, 256 x 192 and 256 x 320 came in, at their older
+// weights: 4.1%), none over 1% slower than those six's pick and the best 1.29
+// times as fast (M 1105, K 3072, N 28672: 231 -> 185 us; M 700, K 3072, N
+// 24576: 116 -> 98).
 struct ScoredTile {
     GemmTile tile;
     int blocksPerCU;
     double weight;
 };
 const ScoredTile kLineTiles[] = {
-    {{256, 384, 512, "e256x384"}, 1, 1.0},  {{256, 256, 512, "e256x256"}, 1, 0.97}, {{256, 288, 768, "e256x288"}, 1, 0.94},
-    {{128, 192, 256, "e128x192"}, 2, 0.92}, {{128, 128, 256, "e128x128"}, 2, 0.87}, {{128, 256, 512, "e128x256"}, 1, 0.75}};
+    {{256, 384, 512, "e256x384"}, 1, 1.0},  {{256, 320, 512, "e256x320"}, 1, 0.98}, {{192, 384, 768, "e192x384"}, 1, 0.92},
+    {{256, 256, 512, "e256x256"}, 1, 0.90}, {{256, 288, 768, "e256x288"}, 1, 0.93}, {{128, 192, 256, "e128x192"}, 2, 0.81},
+    {{256, 192, 512, "e256x192"}, 1, 0.80}, {{192, 256, 768, "e192x256"}, 1, 0.74}, {{128, 128, 256, "e128x128"}, 2, 0.72}};
 
-double lineTileScore(const ScoredTile &t, int64_t m, int64_t n) {
+double lineTileScore(const ScoredTile &t, int64_t m, int64_t n, int64_t k) {
     const int64_t cus = deviceCUs();
     const int64_t tm = cdiv(m, t.tile.bm), tn = cdiv(n, t.tile.bn), tiles = tm * tn;
     const int64_t slots = cus * t.blocksPerCU;
     double fill = (double)tiles / (double)(cdiv(tiles, slots) * slots);
     if (t.blocksPerCU > 1 && tiles <= cus) fill = 0.6 * (double)tiles / (double)cus;
+    else if (t.blocksPerCU > 1 && tiles < slots && m > 512 && k <= 4096) fill *= 0.78;
     const double inside = (double)(m * n) / (double)(tm * t.tile.bm * tn * t.tile.bn);
     return fill * inside * t.weight;
 }
 
-const ScoredTile &bestLineTile(int64_t m, int64_t n) {
+const ScoredTile &bestLineTile(int64_t m, int64_t n, int64_t k) {
     const ScoredTile *best = &kLineTiles[0];
     double bestScore = -1.0;
     for (const ScoredTile &t : kLineTiles) {
-        const double sc = lineTileScore(t, m, n);
+        const double sc = lineTileScore(t, m, n, k);
         if (sc > bestScore) {
             bestScore = sc;
             best = &t;
@@ -951,7 +962,7 @@ GemmPlan gemmSmallPlan(int64_t m, int64_t n, int64_t k, bool maySplit) {
 
 GemmTile gemmTileForm(int64_t m, int64_t n, int64_t k);
 GemmTile gemmTile(int64_t m, int64_t n, int64_t k) {
-    if (!std::getenv("POPCORN_GEMM_TILE") && gemmLinesFit(k, 384)) return bestLineTile(m, n).tile;
+    if (!std::getenv("POPCORN_GEMM_TILE") && gemmLinesFit(k, 384)) return bestLineTile(m, n, k).tile;
     return gemmTileForm(m, n, k);
 }
 
@@ -962,7 +973,9 @@ GemmTile gemmTileForm(int64_t m, int64_t n, int64_t k) {
                                      {128, 128, 256, "e128x128"}, {128, 256, 512, "e128x256"},
                                      {128, 192, 256, "e128x192"}, {256, 384, 512, "e256x384"},
                                      {256, 288, 768, "e256x288"}, {64, 64, 256, "f64x64"},
-                                     {128, 64, 256, "f128x64"},   {128, 128, 256, "f128x128"}};
+                                     {128, 64, 256, "f128x64"},   {128, 128, 256, "f128x128"},
+                                     {256, 320, 512, "e256x320"}, {192, 384, 768, "e192x384"},
+                                     {256, 192, 512, "e256x192"}, {192, 256, 768, "e192x256"}};
     if (const char *e = std::getenv("POPCORN_GEMM_TILE")) {  // tuning override, e.g. "e128x192"
         for (const GemmTile &t : tiles)
             if (std::string(t.suffix) == e && (t.suffix[0] == 'd' ? k % 32 == 0 : gemmOffsetsFit(k, std::max(t.bm, t.bn)))) return t;
@@ -1009,12 +1022,18 @@ int64_t gemmSplitK(int64_t m, int64_t n, int64_t k) {
     for (int64_t s = 2; s <= 8; ++s)
         if ((t384 * s) % cus == 0 && k % (32 * s) == 0 && k / s >= 2048) {
             // with whole-line tiles, split only when it beats the best tile's
-            // score: the split grid fills the CUs, less the share of time its
-            // partials' round trip through HBM adds (8 s bytes per element
-            // at ~7 TB/s against 2 K flop at ~1.2 PFLOP/s: ~700 s / K)
+            // score: the split grid fills the CUs, less its tiles' share
+            // outside C and the share of time that its partials' round trip
+            // through HBM adds (8 s bytes per element at ~7 TB/s against 2 K
+            // flop at ~1.2 PFLOP/s: ~700 s / K). 1.1: the scores rank tiles
+            // over all fills, and a nearly full grid does better than its
+            // score says (f16, unsplit and split: M 2048, N 6144, K 8192: 185
+            // and 205 us, K 14336: 345 and 322; M 512, N 12288, K 8192: 140
+            // and 121; M 375, N 24576, K 4096: 100 and 112)
             if (gemmLinesFit(k, 384)) {
-                const ScoredTile &t = bestLineTile(m, n);
-                if (1.0 - 700.0 * (double)s / (double)k <= lineTileScore(t, m, n)) return 0;
+                const ScoredTile &t = bestLineTile(m, n, k);
+                const double inside = (double)(m * n) / (double)(t384 * 256 * 384);
+                if (inside * (1.0 - 700.0 * (double)s / (double)k) <= 1.1 * lineTileScore(t, m, n, k)) return 0;
             }
             return s;
         }

@@ -31,7 +31,11 @@ def test_small_grid_plan():
     # under 2^29 multiply-adds: one 128 x 128 pass
     assert _names(100, 2304, 2304) == ["matmul_mfma_bf16_bf16_bf16_e128x128"]
     # more than two tiles per CU: the score over the large tiles
-    assert _names(1000, 2304, 9216) == ["matmul_mfma_bf16_bf16_bf16_e128x192"]
+    assert _names(1000, 2304, 9216) == ["matmul_mfma_bf16_bf16_bf16_e256x192"]
+    assert _names(512, 2304, 9216 * 2) == ["matmul_mfma_bf16_bf16_bf16_e128x192"]
+    assert _names(700, 3072, 24576) == ["matmul_mfma_bf16_bf16_bf16_e192x384"]
+    assert _names(4601, 9216, 4096) == ["matmul_mfma_bf16_bf16_bf16_e256x320"]
+    assert _names(2964, 3072, 4096) == ["matmul_mfma_bf16_bf16_bf16_e192x256"]
     # K of whole 16-byte chunks but not whole stages takes the same tiles
     assert _names(190, 2136, 9088)[0].split("_")[-1][0] in "ef"
     # rows too long for a tile's 32-bit offsets, not in whole 64-byte runs
@@ -66,7 +70,8 @@ def env():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile", ["f64x64", "f128x64", "f128x128", "e128x128", "e256x256", "e256x288"])
+@pytest.mark.parametrize("tile", ["f64x64", "f128x64", "f128x128", "e128x128", "e256x256", "e256x288", "e256x320",
+                                  "e192x384", "e256x192", "e192x256"])
 def test_tiles_any_k_integer_exact(env, monkeypatch, tile):
     # 1 to 6 stages (fewer and more than are in flight), the last one whole,
     # or of 1, 2 or 7 chunks; M and N ragged
