@@ -21,9 +21,15 @@
 // each, matching the copy's order (the products' order within a group is
 // free).
 //
-// aq_gemm: a block of 4 waves takes a 128 x 128 tile of C, each wave 64 x 64
-// (2 x 2 MFMA tiles); per group the block copies the X' tile (128 x 64
-// bf16), the packed words, the columns' scale and bias words and the rows'
+// aq_gemm: a block of 4 waves takes a 128 x 128 tile of C, each wave 128 x 32
+// (4 x 1 MFMA tiles), so each packed word is unpacked by one wave only: the
+// vector ALU work (unpacking, the FMAs of s * D) adds to the products' time.
+// Waves of 64 x 64 read fewer fragments but unpack every word twice: 9
+// products back to back, each, M 1000, K 9216, N 2304: 137 -> 124 us; M 2048,
+// K 2304, N 9216: 147 -> 137; M 777: 66 -> 61 (with pauses between them, where
+// the clock is higher: 59.7 -> 59.3, and M 71: 27.0 -> 25.9). Per group the
+// block copies the X' tile (128 x 64 bf16), the packed words, the columns'
+// scale and bias words and the rows'
 // X_g into LDS, three groups in flight (below). Rows past M and columns
 // past N read zeros and are not stored. A block walks its groups one after
 // another, so with few tiles the groups are split over gridDim.y blocks per
@@ -113,7 +119,8 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
     const uint32_t pm = blockIdx.x % nM, pn = blockIdx.x / nM;  // blocks sharing weights run together
     const uint32_t bm = pm * BM, bn = pn * BN;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    constexpr int MI = BM / 32, NI = 1;  // the wave's tiles of 32 x 32
+    const uint32_t wn = wave * 32;
     const uint32_t r = lane & 31, h = lane >> 5;
 
     // buffer resources over whole operands (the host keeps each under 2^31 bytes)
@@ -151,46 +158,46 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    f32x16 acc[2][2];
+    f32x16 acc[MI][NI];
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
+        for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[mi][ni][i] = 0.0f;
 
     // j: the group's index in this block's range; the bias terms of groups
     // j - 1 and j go in one product at odd j, a last even j's alone
-    float px[2] = {0.0f, 0.0f}, pb[2] = {0.0f, 0.0f};  // group j - 1's X_g and b - 128 s
+    float px[MI] = {}, pb[NI] = {};  // group j - 1's X_g and b - 128 s
     auto compute = [&](const uint8_t *stage, uint32_t g, uint32_t j, bool last) {
         const uint8_t *sX = stage, *sW = stage + kXB;
         const uint32_t *sS = reinterpret_cast<const uint32_t *>(stage + kXB + kWB);
         const uint32_t *sB = sS + 128;
         const float *sG = reinterpret_cast<const float *>(stage + kXB + kWB + 1024);
-        // this lane's 4 packed words of each of its two columns: chunks 4 h .. 4 h + 3
-        u32x4 wr[2];
+        // this lane's 4 packed words of its column: chunks 4 h .. 4 h + 3
+        u32x4 wr[NI];
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
+        for (int ni = 0; ni < NI; ++ni) {
             const uint32_t col = wn + ni * 32 + r;
             wr[ni] = *reinterpret_cast<const u32x4 *>(sW + col * 32 + ((h ^ ((col >> 3) & 1)) << 4));
         }
-        f32x16 d[2][2];
+        f32x16 d[MI][NI];
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi)
+        for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-            for (int ni = 0; ni < 2; ++ni)
+            for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) d[mi][ni][i] = 0.0f;
 #pragma unroll
         for (int kk = 0; kk < kGroup / 16; ++kk) {
-            u32x4 a[2], b[2];
+            u32x4 a[MI], b[NI];
 #pragma unroll
-            for (int mi = 0; mi < 2; ++mi) {
-                const uint32_t row = wm + mi * 32 + r, c = 4 * h + kk;
+            for (int mi = 0; mi < MI; ++mi) {
+                const uint32_t row = mi * 32 + r, c = 4 * h + kk;
                 a[mi] = *reinterpret_cast<const u32x4 *>(sX + row * 128 + ((c ^ ((row >> 1) & 7)) << 4));
             }
 #pragma unroll
-            for (int ni = 0; ni < 2; ++ni) {
+            for (int ni = 0; ni < NI; ++ni) {
                 // a packed word gives its values in pair order as 4 bf16 pairs
                 const uint32_t w = wr[ni][kk];
                 b[ni].x = (w & 0x000F000Fu) | kPairBase;
@@ -199,24 +206,24 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
                 b[ni].w = ((w >> 12) & 0x000F000Fu) | kPairBase;
             }
 #pragma unroll
-            for (int mi = 0; mi < 2; ++mi)
+            for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-                for (int ni = 0; ni < 2; ++ni) d[mi][ni] = pk::Mma<pk::BF16>::run(a[mi], b[ni], d[mi][ni]);
+                for (int ni = 0; ni < NI; ++ni) d[mi][ni] = pk::Mma<pk::BF16>::run(a[mi], b[ni], d[mi][ni]);
         }
-        float cs[2], cb[2], cx[2];
+        float cs[NI], cb[NI], cx[MI];
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
+        for (int ni = 0; ni < NI; ++ni) {
             const uint32_t col = wn + ni * 32 + r;
             cs[ni] = bf16_half(sS[col], g);
             const float bias = p.hasBias ? bf16_half(sB[col], g) : 0.0f;
             cb[ni] = bias - 128.0f * cs[ni];
         }
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi) cx[mi] = sG[wm + mi * 32 + r];
+        for (int mi = 0; mi < MI; ++mi) cx[mi] = sG[mi * 32 + r];
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
+        for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-            for (int mi = 0; mi < 2; ++mi)
+            for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[mi][ni][i] = fmaf(cs[ni], d[mi][ni][i], acc[mi][ni][i]);
         // acc += X_g (rows) x (b - 128 s)_g (columns) for two groups at a
@@ -227,23 +234,21 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
         // last group takes k 0 with k 1 zero
         if (!(j & 1)) {
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                px[e] = cx[e];
-                pb[e] = cb[e];
-            }
+            for (int e = 0; e < MI; ++e) px[e] = cx[e];
+#pragma unroll
+            for (int e = 0; e < NI; ++e) pb[e] = cb[e];
         }
         if ((j & 1) || last) {
             const bool pair = (j & 1) != 0;
-            float xa[2], bb[2];
+            float xa[MI], bb[NI];
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                xa[e] = pair ? (h ? cx[e] : px[e]) : (h ? 0.0f : cx[e]);
-                bb[e] = pair ? (h ? cb[e] : pb[e]) : (h ? 0.0f : cb[e]);
-            }
+            for (int e = 0; e < MI; ++e) xa[e] = pair ? (h ? cx[e] : px[e]) : (h ? 0.0f : cx[e]);
 #pragma unroll
-            for (int mi = 0; mi < 2; ++mi)
+            for (int e = 0; e < NI; ++e) bb[e] = pair ? (h ? cb[e] : pb[e]) : (h ? 0.0f : cb[e]);
 #pragma unroll
-                for (int ni = 0; ni < 2; ++ni)
+            for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni)
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[mi], bb[ni], acc[mi][ni], 0, 0, 0);
         }
     };
@@ -269,14 +274,14 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
 
     // C element i of lane l in tile (mi, ni): row (i / 4) * 8 + (l / 32) * 4 + i % 4, column l % 32
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
+        for (int ni = 0; ni < NI; ++ni) {
             const uint32_t col = bn + wn + ni * 32 + r;
             if (col >= N) continue;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const uint32_t m = bm + wm + mi * 32 + (i / 4) * 8 + h * 4 + (i % 4);
+                const uint32_t m = bm + mi * 32 + (i / 4) * 8 + h * 4 + (i % 4);
                 if (m >= M) continue;
                 if constexpr (SPLIT) {
                     P[((uint64_t)blockIdx.y * M + m) * N + col] = acc[mi][ni][i];
