@@ -21,14 +21,23 @@
 //    sits in slot c ^ (2 (k % 8)) so the keys a read touches fall in
 //    different banks.
 // The one-row kernels (flash_decoding_partial_*) run per query row and read
-// K and V Sq times: 21.0 us for the call above, 11.7 here.
+// K and V Sq times: 21.0 us for the call above, 12.1 here (11.7 with weights of
+// one f16 or two bf16, which lost precision, below).
 //
 // Softmax: S^T = K . Q^T, so lane l holds the scores of row l % 16 for keys
 // 4 g + i and 16 + 4 g + i (g = l / 16), already the slots of its P^T
-// operand; maxima and sums run over lanes l, l ^ 16, l ^ 32. Weights enter
-// P.V in the input dtype, bf16 as a high part plus a remainder, and a row's
-// reference max moves only when a score passes it by more than 8 (natural
-// log), as in flash_attention_tiled.hip.
+// operand; maxima and sums run over lanes l, l ^ 16, l ^ 32. A row's
+// reference moves only when a score passes it by more than 8 (natural log),
+// as in flash_attention_tiled.hip.
+//
+// Weights enter P.V with the bits that the one-row kernels' f32 weights have:
+// as the sum of three bf16 (24 bits), or of two f16 (22 bits, and the
+// reference kept 4 octaves below the max, the largest weight 2^15.5, so that
+// the second is rarely subnormal). A score is the sum of partial sums of 32 or
+// 64 products, as a tree over lanes gives them. Relative error of an f32
+// output against 64 bits, 4104 keys, Hd 256: 1.9e-7 from f16 and bf16, as the
+// one-row kernels (1.9e-7); with one f16 1.4e-4, with two bf16 1.7e-6, with a
+// score's products in one chain 2.6e-7.
 #include <type_traits>
 
 #include "mfma.hpp"
@@ -41,8 +50,8 @@ using pk::u32x4;
 
 constexpr int kWaves = 4;
 constexpr int BKV = 32;  // keys per step
-constexpr float kRescaleGap = 8.0f;
 constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+constexpr float kRescaleGap = 8.0f * kLog2e;  // log2 units, as the maxima
 // past every head's range (the host keeps Sk * Hd * 2 below 2^31): zeros
 constexpr int kOutOfRange = (int)0x80000000u;
 
@@ -67,12 +76,14 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
                         float *__restrict__ pO, float *__restrict__ pM, float *__restrict__ pL,
                         typename O::storage *__restrict__ out, const FlashDecodingPartialExtConstants &p) {
     constexpr int KS = HD / 32;                // k-steps of each S^T tile
+    constexpr int kSums = KS == 2 ? 2 : KS / 2;  // partial sums of a score
     constexpr int DT = HD / 16;                // 16-row tiles of O^T
     constexpr int CH = HD / 8;                 // 16-byte chunks per row
     constexpr int kRowsPer = 64 / CH;          // V rows per copy instruction
     constexpr int kCopies = BKV / kRowsPer;    // copy instructions per step
     constexpr int kVary = 8 / kRowsPer;        // distinct chunk swizzles over the instructions
-    constexpr bool kSplitP = std::is_same<T, pk::BF16>::value;
+    constexpr int kParts = std::is_same<T, pk::BF16>::value ? 3 : 2;         // 16-bit terms of a weight
+    constexpr float kLead = std::is_same<T, pk::BF16>::value ? 0.0f : 4.0f;  // max over reference when it moves
     constexpr int LDO = HD + 4;                // merged-state row, in floats
     static_assert(CH <= 64 && kVary >= 1, "a V row is at most one instruction, at least 8 to a swizzle period");
     constexpr int kStage = kWaves * BKV * HD * 2, kMerge = kWaves * 16 * LDO * 4;
@@ -169,14 +180,21 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
             for (int mt = 0; mt < 2; ++mt) {
-                st[rt][mt] = pk::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                pk::f32x4 part[kSums];
 #pragma unroll
-                for (int s = 0; s < KS; ++s) st[rt][mt] = Mma16<T>::run(kf[mt][s], qf[rt][s], st[rt][mt]);
+                for (int c = 0; c < kSums; ++c) {
+                    part[c] = pk::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int s = c * KS / kSums; s < (c + 1) * KS / kSums; ++s) part[c] = Mma16<T>::run(kf[mt][s], qf[rt][s], part[c]);
+                }
+                st[rt][mt] = part[0];
+#pragma unroll
+                for (int c = 1; c < kSums; ++c) st[rt][mt] += part[c];
             }
         __builtin_amdgcn_sched_barrier(0);
         loadK(it + kWaves);
         __builtin_amdgcn_sched_barrier(0);
-        u32x4 pf[RT], pfr[RT];
+        u32x4 pf[RT][kParts];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             float sv[8], mx = -INFINITY, ps = 0.0f, alpha = 1.0f;
@@ -189,10 +207,10 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
                 mx = fmaxf(mx, sv[i]);
             }
             mx = quad16_max(mx) * c2;
-            const bool move = mx > m[rt] + kRescaleGap * kLog2e;
+            const bool move = mx > m[rt] + (kRescaleGap + kLead);
             if (move) {
-                alpha = __builtin_amdgcn_exp2f(m[rt] - mx);
-                m[rt] = mx;
+                alpha = __builtin_amdgcn_exp2f(m[rt] - (mx - kLead));
+                m[rt] = mx - kLead;
             }
             if (__ballot(move)) {
 #pragma unroll
@@ -202,13 +220,16 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
             const float mref = m[rt] == -INFINITY ? 0.0f : m[rt];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float p0 = __builtin_amdgcn_exp2f(fmaf(sv[2 * j], c2, -mref));
-                const float p1 = __builtin_amdgcn_exp2f(fmaf(sv[2 * j + 1], c2, -mref));
+                float p0 = __builtin_amdgcn_exp2f(fmaf(sv[2 * j], c2, -mref));
+                float p1 = __builtin_amdgcn_exp2f(fmaf(sv[2 * j + 1], c2, -mref));
                 ps += p0 + p1;
-                const uint32_t w = pk::pack2<T>(p0, p1);
-                pf[rt][j] = w;
-                if constexpr (kSplitP)
-                    pfr[rt][j] = pk::pack2<T>(p0 - __uint_as_float(w << 16), p1 - __uint_as_float(w & 0xffff0000u));
+#pragma unroll
+                for (int e = 0; e < kParts; ++e) {
+                    const uint32_t w = pk::pack2<T>(p0, p1);
+                    pf[rt][e][j] = w;
+                    p0 -= pk::from_bits16<T>(w & 0xffffu);  // exact
+                    p1 -= pk::from_bits16<T>(w >> 16);
+                }
             }
             l[rt] = l[rt] * alpha + quad16_sum(ps);
         }
@@ -220,8 +241,8 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
             const u32x4 va = {lo.x, lo.y, hi2.x, hi2.y};
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
-                acc[rt][dt] = Mma16<T>::run(va, pf[rt], acc[rt][dt]);
-                if constexpr (kSplitP) acc[rt][dt] = Mma16<T>::run(va, pfr[rt], acc[rt][dt]);
+#pragma unroll
+                for (int e = 0; e < kParts; ++e) acc[rt][dt] = Mma16<T>::run(va, pf[rt][e], acc[rt][dt]);
             }
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // this wave's reads of its V tile are done before it is overwritten
@@ -259,7 +280,6 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
             L += w[v] * sm_l[v][rt * 16 + tr];
         }
         const uint64_t slot = q_row(r) * P + blockIdx.x;
-        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
         for (uint32_t d = td; d < D; d += 64) {
             pk::f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -269,7 +289,7 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
             } else {
                 typename O::storage *dst = out + slot * D + d;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) dst[i] = O::store(o[i] * inv);
+                for (int i = 0; i < 4; ++i) dst[i] = O::store(L > 0.0f ? o[i] / L : 0.0f);  // as the combine
             }
         }
         if (P > 1 && td == 0) {

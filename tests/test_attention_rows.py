@@ -106,3 +106,39 @@ def test_rows_wide_score_range(t):
     enc.encode(_kernel(pa, t, 1, 4, 2, 7, 640, 640, 256, (0, -1), 1.0, upload(pa, q, t), upload(pa, k, t), upload(pa, v, t), out))
     stream.synchronize()
     assert_out(download(out, stream), O.attention_naive(q, k, v, 1.0), EPS[t], t, "wide range")
+
+
+# every kernel of the rule, by a call that takes it
+FORMS = [(1, 4, 2, 4, 300, 64, "d64_r1"), (8, 32, 8, 8, 1030, 64, "d64_r2"), (8, 32, 8, 16, 1030, 64, "d64_r4"),
+         (1, 8, 4, 8, 1500, 128, "d128_r1"), (8, 32, 8, 8, 1030, 128, "d128_r2"), (8, 32, 8, 16, 1030, 128, "d128_r4"),
+         (1, 8, 4, 8, 1500, 256, "d256_r1"), (8, 16, 8, 16, 1030, 256, "d256_r2"), (1, 8, 2, 8, 1500, 512, "d512_r1")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", ["f16", "bf16"])
+@pytest.mark.parametrize("B,Nq,Nkv,Sq,Sk,Hd,form", FORMS)
+def test_rows_hold_f32_precision(t, B, Nq, Nkv, Sq, Sk, Hd, form):
+    # An f32 output against 64 bits. With the weights and every sum in f32 its
+    # error is a handful of roundings of 2^-24 per term (a score, its exponent,
+    # the weight, two products and sums), the terms' own averaged over the
+    # keys: 6e-7 is ten. Weights of one f16 give 1.4e-4, of two bf16 1.7e-6.
+    import oracle as O
+    from gpu_util import download, gpu_env, rounded, upload
+
+    pa, lib, stream, enc = gpu_env()
+    q = rounded(O.normal(Sq, (B, Nq, Sq, Hd)), t)
+    k, v = (rounded(O.normal(Sk + i, (B, Nkv, Sk, Hd)), t) for i in (1, 2))
+    out = upload(pa, np.zeros(q.shape, np.float32), "f32")
+    kern = _kernel(pa, t, B, Nq, Nkv, Sq, Sk, Sk, Hd, (0, -1), None, upload(pa, q, t), upload(pa, k, t), upload(pa, v, t), out)
+    assert kern.function_names[0] == f"flash_attention_rows_{t}_f32_{form}"
+    enc.encode(kern)
+    stream.synchronize()
+    got, err, ref = download(out, stream).astype(np.float64), 0.0, 0.0
+    seen = np.arange(Sk)[None, :] <= np.arange(Sq)[:, None] + Sk - Sq
+    for b in range(min(B, 2)):
+        for h in range(Nq):
+            s = q[b, h].astype(np.float64) @ k[b, h // (Nq // Nkv)].astype(np.float64).T * Hd ** -0.5
+            w = np.where(seen, np.exp(s - s.max()), 0.0)
+            want = w @ v[b, h // (Nq // Nkv)].astype(np.float64) / w.sum(1, keepdims=True)
+            err, ref = err + ((got[b, h] - want) ** 2).sum(), ref + (want ** 2).sum()
+    assert (err / ref) ** 0.5 < 6e-7
