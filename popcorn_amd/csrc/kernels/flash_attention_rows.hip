@@ -30,6 +30,12 @@
 // reference moves only when a score passes it by more than 8 (natural log),
 // as in flash_attention_tiled.hip.
 //
+// A matrix product adds 0 x V for a key that a row does not see, and the terms
+// of one weight have either sign, so where V holds an infinity or a NaN (or a
+// sum passes f32's range) the products give NaN where the sum over the row's
+// own keys does not. A block with such a result runs its rows again on the
+// vector ALUs (fa_rows_seen); finite ones pay one check in the merge.
+//
 // Weights enter P.V with the bits that the one-row kernels' f32 weights have:
 // as the sum of three bf16 (24 bits), or of two f16 (22 bits, and the
 // reference kept 4 octaves below the max, the largest weight 2^15.5, so that
@@ -68,6 +74,57 @@ __device__ inline void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// One row's O, m (log2 units) and l over the keys of [k0, k1) that it sees, in
+// f32 on the vector ALUs with weights of at most 1. 16 lanes per row, lane t's
+// dims 4 t + 64 j; `seen` says which keys.
+template <typename T, int HD, typename Seen>
+__device__ inline void fa_rows_seen(const uint16_t *__restrict__ q, const uint16_t *__restrict__ K,
+                                    const uint16_t *__restrict__ V, uint32_t D, int k0, int k1, float c2, const Seen &seen,
+                                    pk::f32x4 (&o)[HD / 64], float &m, float &l) {
+    constexpr int NJ = HD / 64, U = HD == 512 ? 2 : 4;  // keys in flight
+    const uint32_t td = threadIdx.x % 16 * 4;
+    auto load = [&](const uint16_t *row, int j) {
+        const u32x2 v = td + 64 * j < D ? *reinterpret_cast<const u32x2 *>(row + td + 64 * j) : u32x2{0u, 0u};
+        return pk::f32x4{pk::from_bits16<T>(v.x & 0xffffu), pk::from_bits16<T>(v.x >> 16), pk::from_bits16<T>(v.y & 0xffffu),
+                         pk::from_bits16<T>(v.y >> 16)};
+    };
+    m = -INFINITY, l = 0.0f;
+    pk::f32x4 qv[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        qv[j] = load(q, j);
+        o[j] = pk::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    for (int k = k0; k < k1; k += U) {
+        pk::f32x4 kv[U][NJ], vv[U][NJ];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const uint64_t row = (uint64_t)min(k + u, k1 - 1) * D;
+                kv[u][j] = load(K + row, j);
+                vv[u][j] = load(V + row, j);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s = fmaf(qv[j][i], kv[u][j][i], s);
+            s = pk::group_sum<16>(s) * c2;
+            if (k + u >= k1 || !seen(k + u)) continue;  // a row's lanes together
+            const float mn = fmaxf(m, s);
+            if (mn == -INFINITY) continue;
+            const float alpha = __builtin_amdgcn_exp2f(m - mn), w = __builtin_amdgcn_exp2f(s - mn);
+            l = l * alpha + w;
+            m = mn;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) o[j] = o[j] * alpha + vv[u][j] * w;
+        }
+    }
+}
+
 // pO [rows][P][Hd], pM, pL [rows][P] (rows as in q: b, head, query) for the
 // LSE combine (flash_decoding_reduce_*_ext; m in natural-log units), or with
 // P = 1 the output itself.
@@ -89,6 +146,8 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
     constexpr int kStage = kWaves * BKV * HD * 2, kMerge = kWaves * 16 * LDO * 4;
     __shared__ __attribute__((aligned(16))) uint8_t smem[kStage > kMerge ? kStage : kMerge];
     __shared__ float sm_m[kWaves][RT * 16], sm_l[kWaves][RT * 16];
+    __shared__ uint32_t sm_bad;
+    if (threadIdx.x == 0) sm_bad = 0;  // written and read behind the merge's barriers
 
     const uint32_t lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -118,8 +177,11 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
     const int kLo = p.maskKind == 1u ? max(0, first - p.slidingWindow + 1) : 0;
     const int kHi = p.maskKind == 2u ? (int)p.Sk : min((int)p.Sk, last + 1);
     const uint32_t n = kHi > kLo ? (uint32_t)(kHi - kLo + BKV - 1) / BKV : 0u;
-    const uint32_t hi = (uint32_t)((uint64_t)n * (blockIdx.x + 1) / P);
-    uint32_t it = (uint32_t)((uint64_t)n * blockIdx.x / P) + wave;
+    const uint32_t lo = (uint32_t)((uint64_t)n * blockIdx.x / P), hi = (uint32_t)((uint64_t)n * (blockIdx.x + 1) / P);
+    uint32_t it = lo + wave;
+    auto allowed = [&](int key, int pos) {
+        return (key < (int)p.Sk) & ((p.maskKind == 2u) | (key <= pos)) & ((p.maskKind != 1u) | (pos - key < p.slidingWindow));
+    };
 
     const __amdgpu_buffer_rsrc_t rsK = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(K + kvoff), 0,
                                                                           (int)(p.Sk * D * 2), 0x00020000);
@@ -201,9 +263,7 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int key = k0 + (i / 4) * 16 + (int)g * 4 + i % 4;
-                const bool ok = (key < (int)p.Sk) & ((p.maskKind == 2u) | (key <= posQ[rt])) &
-                                ((p.maskKind != 1u) | (posQ[rt] - key < p.slidingWindow));
-                sv[i] = ok ? st[rt][i / 4][i % 4] : -INFINITY;
+                sv[i] = allowed(key, posQ[rt]) ? st[rt][i / 4][i % 4] : -INFINITY;
                 mx = fmaxf(mx, sv[i]);
             }
             mx = quad16_max(mx) * c2;
@@ -261,6 +321,22 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
     }
     float *sO = reinterpret_cast<float *>(smem);
     const uint32_t tr = threadIdx.x / 16, td = threadIdx.x % 16 * 4;
+    auto store4 = [&](uint64_t slot, uint32_t d, const pk::f32x4 &o, float L) {
+        if (P > 1) {
+            *reinterpret_cast<pk::f32x4 *>(pO + slot * D + d) = o;
+        } else {
+            typename O::storage *dst = out + slot * D + d;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[i] = O::store(L > 0.0f ? o[i] / L : 0.0f);  // as the combine
+        }
+    };
+    auto storeML = [&](uint64_t slot, float M, float L) {
+        if (P > 1 && td == 0) {
+            pM[slot] = M * kLn2;
+            pL[slot] = L;
+        }
+    };
+    bool bad = false;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         __syncthreads();  // V tiles and the previous tile's state are read
@@ -284,18 +360,26 @@ __device__ void fa_rows(const uint16_t *__restrict__ Q, const uint16_t *__restri
             pk::f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int v = 0; v < kWaves; ++v) o += *reinterpret_cast<const pk::f32x4 *>(&sO[(v * 16 + tr) * LDO + d]) * w[v];
-            if (P > 1) {
-                *reinterpret_cast<pk::f32x4 *>(pO + slot * D + d) = o;
-            } else {
-                typename O::storage *dst = out + slot * D + d;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) dst[i] = O::store(L > 0.0f ? o[i] / L : 0.0f);  // as the combine
-            }
+            for (int i = 0; i < 4; ++i) bad |= !(fabsf(o[i]) < INFINITY);
+            store4(slot, d, o, L);
         }
-        if (P > 1 && td == 0) {
-            pM[slot] = M * kLn2;
-            pL[slot] = L;
-        }
+        storeML(slot, M, L);
+    }
+    if (bad) sm_bad = 1;
+    __syncthreads();
+    if (!sm_bad) return;
+    for (uint32_t r = r0 + tr; r < min(r0 + 16 * RT, R); r += 16) {
+        const int pos = (int)p.Sk - (int)p.Sq + (int)(r / G);
+        pk::f32x4 o[HD / 64];
+        float M, L;
+        fa_rows_seen<T, HD>(Q + q_row(r) * D, K + kvoff, V + kvoff, D, kLo + (int)(lo * BKV),
+                            min(kLo + (int)(hi * BKV), (int)p.Sk), c2, [&](int key) { return allowed(key, pos); }, o, M, L);
+        const uint64_t slot = q_row(r) * P + blockIdx.x;
+#pragma unroll
+        for (int j = 0; j < HD / 64; ++j)
+            if (td + 64 * j < D) store4(slot, td + 64 * j, o[j], L);
+        storeML(slot, M, L);
     }
 }
 

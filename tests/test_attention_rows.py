@@ -108,6 +108,22 @@ def test_rows_wide_score_range(t):
     assert_out(download(out, stream), O.attention_naive(q, k, v, 1.0), EPS[t], t, "wide range")
 
 
+def _own_keys(q, k, v, scale, mask=(0, -1)):
+    """Attention in 64 bits, each row over the keys it sees and no others."""
+    B, Nq, Sq, Hd = q.shape
+    Nkv, Sk = k.shape[1:3]
+    out = np.zeros(q.shape)
+    with np.errstate(all="ignore"):  # the tests put infinities and NaN in K and V
+        for b, h, i in np.ndindex(B, Nq, Sq):
+            pos = Sk - Sq + i
+            lo = max(0, pos - mask[1] + 1) if mask[0] == 1 else 0
+            kk, vv = (x[b, h // (Nq // Nkv), lo:pos + 1].astype(np.float64) for x in (k, v))
+            s = kk @ q[b, h, i].astype(np.float64) * scale
+            w = np.exp(s - s.max())
+            out[b, h, i] = w @ vv / w.sum()
+    return out
+
+
 # every kernel of the rule, by a call that takes it
 FORMS = [(1, 4, 2, 4, 300, 64, "d64_r1"), (8, 32, 8, 8, 1030, 64, "d64_r2"), (8, 32, 8, 16, 1030, 64, "d64_r4"),
          (1, 8, 4, 8, 1500, 128, "d128_r1"), (8, 32, 8, 8, 1030, 128, "d128_r2"), (8, 32, 8, 16, 1030, 128, "d128_r4"),
@@ -133,12 +149,44 @@ def test_rows_hold_f32_precision(t, B, Nq, Nkv, Sq, Sk, Hd, form):
     assert kern.function_names[0] == f"flash_attention_rows_{t}_f32_{form}"
     enc.encode(kern)
     stream.synchronize()
-    got, err, ref = download(out, stream).astype(np.float64), 0.0, 0.0
-    seen = np.arange(Sk)[None, :] <= np.arange(Sq)[:, None] + Sk - Sq
-    for b in range(min(B, 2)):
-        for h in range(Nq):
-            s = q[b, h].astype(np.float64) @ k[b, h // (Nq // Nkv)].astype(np.float64).T * Hd ** -0.5
-            w = np.where(seen, np.exp(s - s.max()), 0.0)
-            want = w @ v[b, h // (Nq // Nkv)].astype(np.float64) / w.sum(1, keepdims=True)
-            err, ref = err + ((got[b, h] - want) ** 2).sum(), ref + (want ** 2).sum()
-    assert (err / ref) ** 0.5 < 6e-7
+    want = _own_keys(q[:2], k[:2], v[:2], Hd ** -0.5)
+    err = download(out, stream)[:2].astype(np.float64) - want
+    assert np.linalg.norm(err) / np.linalg.norm(want) < 6e-7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", ["f16", "bf16"])
+@pytest.mark.parametrize("B,Nq,Nkv,Sq,Sk,Hd,form", FORMS)
+def test_rows_non_finite_values(t, B, Nq, Nkv, Sq, Sk, Hd, form):
+    # infinities and NaN in the K and V of single keys change only the rows
+    # that see them: K of NaN at the last key (only the last query sees it), V of
+    # NaN at the one before, and an infinity of V in the middle of the cache,
+    # which every row sees; with a window, those before it change no row
+    import oracle as O
+    from conftest import assert_out
+    from gpu_util import EPS, download, gpu_env, rounded, upload
+
+    pa, lib, stream, enc = gpu_env()
+    q = rounded(O.normal(Sq, (B, Nq, Sq, Hd)), t)
+    k, v = (rounded(O.normal(Sk + i, (B, Nkv, Sk, Hd)), t) for i in (1, 2))
+    first = Sk - Sq  # the first query's own key
+    for mask in ((0, -1), (1, 70)):
+        kk, vv = k.copy(), v.copy()
+        kk[:, :, Sk - 1], vv[:, :, Sk - 2] = np.nan, np.nan
+        if mask[0] == 0:
+            vv[:, :, 40, Hd - 3] = np.inf
+        else:
+            vv[:, :, first - 70], kk[:, :, first - 71], vv[:, :, first - 75] = -np.inf, np.nan, np.nan
+            vv[:, :, first - 5, 1] = -np.inf  # inside every window
+        out = upload(pa, np.zeros(q.shape, np.float32), t)
+        kern = _kernel(pa, t, B, Nq, Nkv, Sq, Sk, Sk, Hd, mask, None, upload(pa, q, t), upload(pa, kk, t), upload(pa, vv, t), out)
+        name = kern.function_names[0]
+        assert name.startswith(f"flash_attention_rows_{t}_{t}_d{Hd}_") and (mask[0] or name.endswith(form))
+        enc.encode(kern)
+        stream.synchronize()
+        got, ref = download(out, stream)[:2, :, :-1], _own_keys(q[:2], kk[:2], vv[:2], Hd ** -0.5, mask)[:, :, :-1]
+        assert np.isfinite(ref[:, :, 0, 2]).all() and np.isnan(ref[:, :, -1]).all() and np.isinf(ref[:, :, 0]).any()
+        for same in (np.isnan, np.isposinf, np.isneginf):
+            np.testing.assert_array_equal(same(got), same(ref), err_msg=f"{name} {mask} {same.__name__}")
+        ok = np.isfinite(ref)
+        assert_out(got[ok], ref[ok], EPS[t], t, f"{name} {mask}")
