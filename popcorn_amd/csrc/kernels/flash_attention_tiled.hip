@@ -1265,15 +1265,18 @@ __device__ void fa_split_merge(const float *__restrict__ pO, const float *__rest
         for (uint32_t j0 = 0; j0 < n; j0 += 8) {
             float4 a[8];
 #pragma unroll
-            for (uint32_t j = 0; j < 8; ++j)  // past the last part: that part again, with no weight
+            for (uint32_t j = 0; j < 8; ++j)  // past the last part: that part again, not added
                 a[j] = *reinterpret_cast<const float4 *>(po + (uint64_t)(i0 + min(j0 + j, n - 1)) * BQ * HD);
 #pragma unroll
             for (uint32_t j = 0; j < 8; ++j) {
-                const float wj = j0 + j < n ? __shfl(w, (int)(j0 + j), (int)kLanes) : 0.0f;
-                o.x += wj * a[j].x;
-                o.y += wj * a[j].y;
-                o.z += wj * a[j].z;
-                o.w += wj * a[j].w;
+                // a select of both: the part's infinity times a weight of 0 is a
+                // NaN, and behind a branch the loads above would sink to it
+                const bool part = j0 + j < n;
+                const float wj = part ? __shfl(w, (int)(j0 + j), (int)kLanes) : 0.0f;
+                o.x += wj * (part ? a[j].x : 0.0f);
+                o.y += wj * (part ? a[j].y : 0.0f);
+                o.z += wj * (part ? a[j].z : 0.0f);
+                o.w += wj * (part ? a[j].w : 0.0f);
             }
         }
     }

@@ -74,3 +74,30 @@ def test_runs_vs_oracle(t, B, Nq, Nkv, Sq, Sk, cap, Hd, mask):
     pa.KernelCommandEncoder(lib, stream, Empty()).encode(kern)
     stream.synchronize()
     assert_out(download(out, stream), ref, EPS[t], t, "whole tiles")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hd", [64, 128, 256])
+def test_infinite_value_stays_infinite(Hd):
+    # an infinity in V at the last key, which every row sees, in the last run
+    # of each tile: the dims it reaches are infinite, no dim is a NaN. Queries
+    # of 0 weigh every key alike, so the rest are the keys' mean.
+    import oracle as O
+    from gpu_util import download, gpu_env, rounded, upload
+
+    pa, lib, stream, enc = gpu_env()
+    B, Nq, Nkv, Sq, Sk = 1, 4, 2, 40, 2000
+    k, v = (rounded(O.normal(Sk + i, (B, Nkv, Sk, Hd)), "f16") for i in (1, 2))
+    v[..., Sk - 1, 3], v[..., Sk - 1, Hd - 1] = np.inf, -np.inf
+    q = np.zeros((B, Nq, Sq, Hd), np.float32)
+    out = upload(pa, q, "f16")
+    kern = _kernel(pa, "f16", B, Nq, Nkv, Sq, Sk, Sk, Hd, (2, -1), upload(pa, q, "f16"), upload(pa, k, "f16"), upload(pa, v, "f16"), out)
+    assert len(kern.function_names) == 2 and kern.function_names[1].startswith("flash_attention_split_merge_")
+    enc.encode(kern)
+    stream.synchronize()
+    got = download(out, stream)
+    want = np.repeat(v.astype(np.float64).mean(2), Nq // Nkv, 1)[:, :, None].repeat(Sq, 2)
+    assert np.isposinf(got[..., 3]).all() and np.isneginf(got[..., Hd - 1]).all()
+    ok = np.isfinite(want)
+    # means of 2000 values under 5: f32 sums and one rounding to f16, of a unit of 2^-11 at 0.15 at most
+    assert ok.sum() == want.size // Hd * (Hd - 2) and np.abs(got[ok] - want[ok]).max() < 2e-4
