@@ -234,7 +234,7 @@ public:
     std::string describe() const override {
         if (path_ == Kernels::AttentionPath::tiled)
             return runLength_ || (nSplit_ && !mergedPairs()) ? tiledName_ + "," + mergeName_ : tiledName_;
-        if (rowTiles_) return rowsP_ > 1 ? rowsName_ + "," + reduceName_ : rowsName_;
+        if (rowTiles_) return rowsName_ + std::to_string(rowTiles_) + (rowsP_ > 1 ? "," + reduceName_ : std::string());
         return partialName_ + "," + reduceName_;
     }
 
@@ -261,11 +261,21 @@ public:
             c.kvStride = (uint32_t)d_.cap;
             c.splitFrom = (uint32_t)(c.qTilesPerHead - nSplit_);
             c.pairTiles = pairTiles_ ? (mergedPairs() ? 2u : 1u) : 0u;
-            if (runLength_ && encodeRuns(enc, c)) return;
+            int64_t nSplit = nSplit_;
+            if (runLength_) {
+                if (encodeRuns(enc, c)) return;
+                // no scratch: pairs, whose exchange the stream keeps (made
+                // here unless the stream is captured), else whole tiles
+                if (!mergedPairs() || (enc.capturing() && !pairExchangeHeld(enc.stream(), pairBytes()))) {
+                    nSplit = 0;
+                    c.splitFrom = c.qTilesPerHead;
+                    c.pairTiles = 0;
+                }
+            }
             // one block per tile; a split tile's two halves take two, a pair
             // of tiles two in all
-            const int64_t items = d_.B * d_.Nq * ((int64_t)c.qTilesPerHead + (pairTiles_ ? 0 : nSplit_));
-            if (!nSplit_) {
+            const int64_t items = d_.B * d_.Nq * ((int64_t)c.qTilesPerHead + (c.pairTiles ? 0 : nSplit));
+            if (!nSplit) {
                 // no split tile: the partial-state arguments are never touched
                 FixedDispatch fa(tiledName_,
                                  {{q_, kRead}, {k_, kRead}, {v_, kRead}, {out_, kWrite}, {q_, kRead}, {q_, kRead},
@@ -281,7 +291,7 @@ public:
                 // merges, so no merge kernel
                 const int64_t tiles = d_.B * d_.Nq * nSplit_;
                 const size_t oBytes = (size_t)(tiles * 128 * hdp_) * 4;
-                const PairExchange &x = pairExchange(enc.stream(), oBytes + (size_t)(tiles * 128 * 2) * 4);
+                const PairExchange &x = pairExchange(enc.stream(), pairBytes());
                 const uint64_t ticket = nextTicket();
                 c.ticketLo = (uint32_t)ticket;
                 c.ticketHi = (uint32_t)(ticket >> 32);
@@ -323,8 +333,7 @@ public:
     }
 
     // Runs of key steps: O, then (m, l), of every run's 128 rows in one scratch
-    // buffer. False, and nothing encoded, without it: the whole or paired
-    // tiles need none.
+    // buffer. False, and nothing encoded, without it.
     bool encodeRuns(KernelCommandEncoder &enc, TiledFlashAttentionConstants c) const {
         const int64_t BH = d_.B * d_.Nq, rows = BH * runsPerHead_ * 128;
         return enc.tryTemporaryTensor(ScratchSpec{{rows, hdp_ + 2}, DataType::f32}, [&](Tensor part) {
@@ -387,15 +396,16 @@ public:
     }
 
     // A few query rows on the matrix cores: the partial states of rowsP_
-    // partitions and their combine, or without scratch for them one partition.
+    // partitions and their combine, or without scratch for them one partition,
+    // of one row tile per block so that there are as many blocks as there can be.
     void encodeRows(KernelCommandEncoder &enc) const {
         const int64_t rows = d_.B * d_.Nq * d_.Sq, slots = rows * rowsP_;
-        auto launch = [&](int64_t P, const Tensor &pO, const Tensor &pM, const Tensor &pL) {
+        auto launch = [&](int64_t rowTiles, int64_t P, const Tensor &pO, const Tensor &pM, const Tensor &pL) {
             DispatchSize ds;
-            ds.grid = dim3((unsigned)P, (unsigned)(d_.B * d_.Nkv * cdiv(d_.Sq * (d_.Nq / d_.Nkv), 16 * rowTiles_)), 1);
+            ds.grid = dim3((unsigned)P, (unsigned)(d_.B * d_.Nkv * cdiv(d_.Sq * (d_.Nq / d_.Nkv), 16 * rowTiles)), 1);
             ds.block = dim3(kBlock, 1, 1);
             // with one partition the output is written and the partials are not; else the other way round
-            FixedDispatch fa(rowsName_,
+            FixedDispatch fa(rowsName_ + std::to_string(rowTiles),
                              {{q_, kRead}, {k_, kRead}, {v_, kRead}, {pO, P > 1 ? kWrite : kRead},
                               {pM, P > 1 ? kWrite : kRead}, {pL, P > 1 ? kWrite : kRead}, {out_, kWrite}},
                              {bytesOf(partialConstants(P))}, ds);
@@ -406,11 +416,11 @@ public:
                 Tensor pO(base, Shape({slots, d_.Hd}), DataType::f32);
                 Tensor pM(base + slots * d_.Hd, Shape({slots}), DataType::f32);
                 Tensor pL(base + slots * (d_.Hd + 1), Shape({slots}), DataType::f32);
-                launch(rowsP_, pO, pM, pL);
+                launch(rowTiles_, rowsP_, pO, pM, pL);
                 encodeReduce(enc, pO, pM, pL, rowsP_);
             }))
             return;
-        launch(1, q_, q_, q_);
+        launch(rowsP_ > 1 ? 1 : rowTiles_, 1, q_, q_, q_);
     }
 
     FlashDecodingPartialExtConstants partialConstants(int64_t P) const {
@@ -491,7 +501,7 @@ private:
         while (rowTiles_ > 1 && (R <= 8 * rowTiles_ || blocks(rowTiles_) * cdiv(steps, 8) < cus)) rowTiles_ /= 2;
         rowsP_ = steps <= 12 ? 1 : std::clamp<int64_t>(cus / blocks(rowTiles_), 1, cdiv(steps, 4));
         rowsName_ = std::string("flash_attention_rows_") + tag(t) + "_" + tag(out_.dataType) + "_d" + std::to_string(hdp) +
-                    "_r" + std::to_string(rowTiles_);
+                    "_r";
     }
 
     // Runs (pairTiles 3): calls whose tiles leave CUs idle cut every tile's
@@ -590,7 +600,7 @@ private:
     bool pairTiles_ = false;
     int64_t runLength_ = 0, runsPerHead_ = 0;  // runs of key steps (0: none)
     int64_t rowTiles_ = 0, rowsP_ = 1;         // a few rows on the matrix cores (0: not)
-    std::string rowsName_;
+    std::string rowsName_;                     // up to its number of row tiles
     bool rows16_ = false;  // the 16-rows-per-wave kernel: 8 waves per 128-row tile (4 per 64 at Hd 512 and in f32)
     int64_t hdp_ = 0;      // the tiled kernel's head dim: Hd padded to 64, 128, 256 or 512
     bool tiles64() const { return hdp_ == 512 || q_.dataType == DataType::f32; }
@@ -601,6 +611,8 @@ private:
     // Paired tiles are merged inside the tiled kernels (pairTiles 2).
     bool pairMergeInKernel_ = true;
     bool mergedPairs() const { return pairTiles_ && pairMergeInKernel_; }
+    // Merged pairs' published parts: O, then (m, l), of each split tile's 128 rows.
+    size_t pairBytes() const { return (size_t)(d_.B * d_.Nq * nSplit_ * 128 * (hdp_ + 2)) * 4; }
     // A 64-bit value, never 0 or ~0 and distinct per launch, for the ready flags
     // of merged pairs: a counter, started from the clock so that processes
     // differ, through the splitmix64 finaliser.
@@ -1041,9 +1053,8 @@ int64_t gemmSplitK(int64_t m, int64_t n, int64_t k) {
 }
 
 // The split-K GEMM: f32 partial products per split in scratch, then one
-// pass that sums them and rounds to C's dtype. Without scratch (none to be
-// had, or a capture that would have to allocate it) the whole product runs on
-// unsplit tiles.
+// pass that sums them and rounds to C's dtype. Without scratch the whole
+// product runs on unsplit tiles.
 class SplitKMatmulKernel : public Kernel {
 public:
     SplitKMatmulKernel(const Tensor &a, const Tensor &b, const Tensor &c, int64_t m, int64_t k, int64_t n, GemmPlan plan)
@@ -2377,6 +2388,15 @@ PairExchange &pairExchange(hipStream_t stream, size_t dataBytes) {
         x.dataBytes = n;
     }
     return x;
+}
+
+bool pairExchangeHeld(hipStream_t stream, size_t dataBytes) {
+    int dev = 0;
+    checkHip(hipGetDevice(&dev), "hipGetDevice");
+    auto &r = pairRegistry();
+    std::lock_guard<std::mutex> g(r.mu);
+    const auto it = r.byStream.find({dev, stream});
+    return it != r.byStream.end() && it->second.flags && it->second.dataBytes >= dataBytes;
 }
 
 void checkPairExchange(hipStream_t stream, bool allStreams) {

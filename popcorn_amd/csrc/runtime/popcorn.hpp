@@ -121,9 +121,6 @@ public:
     virtual ~KernelScratchAllocator() = default;
     virtual KernelTemporaryBuffer borrowTemporaryBuffer(size_t length) = 0;
     virtual void releaseTemporaryBuffer(const KernelTemporaryBuffer &) {}
-    // Whether a borrow of `length` bytes would be served from memory already
-    // held (false where that is not known).
-    virtual bool holds(size_t length) const { return false; }
 };
 
 // Best-fit pool over hipMalloc'd buffers for one stream (the GemmaCLI
@@ -133,7 +130,6 @@ public:
     ~ScratchPool() override;
     KernelTemporaryBuffer borrowTemporaryBuffer(size_t length) override;
     void releaseTemporaryBuffer(const KernelTemporaryBuffer &t) override;
-    bool holds(size_t length) const override;
     size_t bytes() const;
 
 private:
@@ -275,11 +271,11 @@ public:
     }
 
     // The same for work that can also be done without the scratch: false, and
-    // nothing done, where the allocator has none to give or, while the stream
-    // is being captured, would have to allocate it.
+    // nothing done, where the allocator has none to give. While the stream is
+    // captured the same borrow decides (it may allocate then, as the pool
+    // does), so a graph holds the kernels that the eager call runs.
     template <typename F>
     bool tryTemporaryTensor(const ScratchSpec &spec, F &&body) {
-        if (capturing() && !scratch_.holds(spec.byteCount())) return false;
         KernelTemporaryBuffer t;
         try {
             t = scratch_.borrowTemporaryBuffer(spec.byteCount());
@@ -292,6 +288,7 @@ public:
 
     KernelLibrary &library() { return library_; }
     hipStream_t stream() const { return stream_; }
+    bool capturing() const;  // the stream is being captured into a graph
     popcorn_encoder_stats_t stats() const;
     // When set, dispatch() launches only kernels with this function name and
     // skips the rest (used to time one kernel of a composite sequence).
@@ -315,7 +312,6 @@ private:
         } release{scratch_, t};
         body(Tensor(t.buffer, Shape(spec.shape), spec.dataType));
     }
-    bool capturing() const;
     bool needsBarrier(const std::vector<Binding> &bindings) const;
     void recordAccesses(const std::vector<Binding> &bindings);
 
@@ -492,6 +488,8 @@ struct PairExchange {
 // The exchange of `stream` on the current device with at least `dataBytes`
 // of data.
 PairExchange &pairExchange(hipStream_t stream, size_t dataBytes);
+// Whether pairExchange(stream, dataBytes) would allocate nothing.
+bool pairExchangeHeld(hipStream_t stream, size_t dataBytes);
 // After `stream` has drained (or, with stream == nullptr and allStreams,
 // every stream of the current device): throws -1019 when a merged pair's
 // wait gave up since the last check, clearing that exchange's flags first.

@@ -108,6 +108,21 @@ size_t ScratchSpec::byteCount() const {
 
 // ---- scratch -------------------------------------------------------------------
 
+namespace {
+
+// Lets this thread allocate device memory while a stream is captured: in the
+// other capture modes hipMalloc fails and ends the capture.
+class RelaxedCapture {
+public:
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;  // then the thread's own
+};
+
+}  // namespace
+
 ScratchPool::~ScratchPool() {
     for (auto &kv : all_) (void)hipFree(kv.first);
 }
@@ -123,6 +138,7 @@ KernelTemporaryBuffer ScratchPool::borrowTemporaryBuffer(size_t length) {
     }
     size_t rounded = (length + 255) & ~(size_t)255;
     void *p = nullptr;
+    RelaxedCapture relaxed;
     if (hipMalloc(&p, rounded) != hipSuccess) {
         (void)hipGetLastError();
         throw Error::tensorAllocationFailed(rounded);
@@ -138,11 +154,6 @@ void ScratchPool::releaseTemporaryBuffer(const KernelTemporaryBuffer &t) {
     if (it != all_.end()) free_.emplace(it->second, t.buffer);
 }
 
-bool ScratchPool::holds(size_t length) const {
-    std::lock_guard<std::mutex> g(mu_);
-    return free_.lower_bound(std::max<size_t>(length, 1)) != free_.end();
-}
-
 size_t ScratchPool::bytes() const {
     std::lock_guard<std::mutex> g(mu_);
     return bytes_;
@@ -151,6 +162,7 @@ size_t ScratchPool::bytes() const {
 KernelTemporaryBuffer CScratchAllocator::borrowTemporaryBuffer(size_t length) {
     void *p = nullptr;
     int32_t reused = 0;
+    RelaxedCapture relaxed;  // a caller's allocator may call hipMalloc too
     popcorn_status_t st = a_.borrow(a_.context, std::max<size_t>(length, 1), &p, &reused);
     if (st != POPCORN_OK || !p) throw Error(st ? st : POPCORN_ERR_TENSOR_ALLOCATION_FAILED, "scratch allocator failed to borrow " + std::to_string(length) + " bytes");
     return KernelTemporaryBuffer{p, length, reused != 0};
