@@ -254,7 +254,11 @@ popcorn_status_t popcorn_launch(popcorn_stream_t stream, popcorn_function_t func
 /* ---- scratch (KernelResources.swift:5-36, ScratchSpec.swift:10-26) ------- */
 
 /* KernelScratchAllocator: borrow returns device memory of >= length bytes and
- * whether it may hold earlier writes (KernelTemporaryBuffer.wasReused). */
+ * whether it may hold earlier writes (KernelTemporaryBuffer.wasReused). With
+ * nothing to give it returns -1003, -1011, -1012, -1013 or a null buffer:
+ * kernels that can do without the scratch then run without it, the others fail
+ * with that status, as all do with any other status. It may be called while
+ * the encoder's stream is captured, and may call hipMalloc then. */
 typedef struct {
     void *context;
     popcorn_status_t (*borrow)(void *context, size_t length, void **buffer, int32_t *was_reused);

@@ -33,6 +33,11 @@ class Error : public std::exception {
 public:
     Error(int32_t code, std::string message) : code_(code), message_(std::move(message)) {}
     int32_t code() const { return code_; }
+    // There is no memory to be had, of the kinds an allocator reports.
+    bool outOfMemory() const {
+        return code_ == POPCORN_ERR_TENSOR_ALLOCATION_FAILED || code_ == POPCORN_ERR_HEAP_ALLOCATION_FAILED ||
+               code_ == POPCORN_ERR_WORKSPACE_EXHAUSTED || code_ == POPCORN_ERR_GPU_OUT_OF_MEMORY;
+    }
     const char *what() const noexcept override { return message_.c_str(); }
 
     static Error kernelFunctionNotFound(const std::string &name);
@@ -231,7 +236,8 @@ public:
     virtual ~Kernel() = default;
     virtual std::vector<Binding> tensors() const = 0;
     virtual void encode(KernelCommandEncoder &encoder) const = 0;
-    // Function names this kernel dispatches, in order ("a,b").
+    // Function names this kernel dispatches, in order ("a,b"), given the scratch
+    // that its plan borrows.
     virtual std::string describe() const = 0;
 };
 
@@ -271,7 +277,8 @@ public:
     }
 
     // The same for work that can also be done without the scratch: false, and
-    // nothing done, where the allocator has none to give. While the stream is
+    // nothing done, where the allocator has none to give (any other error of
+    // it is the caller's to see). While the stream is
     // captured the same borrow decides (it may allocate then, as the pool
     // does), so a graph holds the kernels that the eager call runs.
     template <typename F>
@@ -279,7 +286,8 @@ public:
         KernelTemporaryBuffer t;
         try {
             t = scratch_.borrowTemporaryBuffer(spec.byteCount());
-        } catch (const Error &) {
+        } catch (const Error &e) {
+            if (!e.outOfMemory()) throw;
             return false;
         }
         withBuffer(t, spec, body);

@@ -426,7 +426,13 @@ class ScratchPool:
 
 
 class KernelScratchAllocator:
-    """Base for Python allocators: override borrow(length) -> (ptr, was_reused) and release(ptr)."""
+    """Base for Python allocators: override borrow(length) -> (ptr, was_reused) and release(ptr).
+
+    A borrow that has nothing to give raises MemoryError (or the PopcornError of a
+    failed allocation): kernels that can do without the scratch then run without
+    it. Any other exception ends the encode, as the cause of its PopcornError."""
+
+    error = None  # what the last failed borrow raised
 
     def borrow(self, length: int):
         raise NotImplementedError
@@ -442,8 +448,11 @@ class KernelScratchAllocator:
                 if reused:
                     reused[0] = 1 if was_reused else 0
                 return 0
-            except Exception:
-                return PopcornError.TENSOR_ALLOCATION_FAILED
+            except Exception as e:
+                self.error = e
+                if isinstance(e, PopcornError):
+                    return e.code
+                return PopcornError.TENSOR_ALLOCATION_FAILED if isinstance(e, MemoryError) else PopcornError.GPU_INTERNAL
 
         def _release(ctx, ptr):
             self.release(ptr)
@@ -731,11 +740,16 @@ class KernelCommandEncoder:
                 flat.extend(x for x in k if x is not None)
             elif k is not None:
                 flat.append(k)
-        if len(flat) == 1:
-            check(lib().popcorn_encoder_encode(self.handle, flat[0].handle))
-        elif flat:
-            arr = (C.c_void_p * len(flat))(*[k.handle for k in flat])
-            check(lib().popcorn_encoder_encode_all(self.handle, arr, len(flat)))
+        if isinstance(self._scratch, KernelScratchAllocator):
+            self._scratch.error = None
+        try:
+            if len(flat) == 1:
+                check(lib().popcorn_encoder_encode(self.handle, flat[0].handle))
+            elif flat:
+                arr = (C.c_void_p * len(flat))(*[k.handle for k in flat])
+                check(lib().popcorn_encoder_encode_all(self.handle, arr, len(flat)))
+        except PopcornError as e:
+            raise e from getattr(self._scratch, "error", None)
 
     def barrier(self) -> None:
         check(lib().popcorn_encoder_barrier(self.handle))

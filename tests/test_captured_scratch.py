@@ -1,7 +1,8 @@
 """Kernels whose plan wants scratch but does not need it (16-bit Matmul split
 over K, attention of a few rows, attention in runs of key steps), recorded in a
 HIP graph: with any allocator that gives scratch, warm or cold, the graph holds
-the kernels of the plan, and its replays equal the eager call."""
+the kernels of the plan, and its replays equal the eager call; and the errors
+of an allocator."""
 import ctypes as C
 import os
 import sys
@@ -157,3 +158,32 @@ def test_graph_without_scratch(env, call, eager):
         # the same sums in another order: a bf16 unit in the last place apart at most, or under the smallest normal result
         np.testing.assert_allclose(got, ref, rtol=2.0 ** -7, atol=1e-4)
     _hip("hipGraphExecDestroy", graph)
+
+
+def test_allocator_errors(env):
+    # no memory: the kernels that can do without it run; any other error of the
+    # allocator reaches the caller, with what it raised
+    pa, lib, stream, _ = env
+
+    class Failing(pa.KernelScratchAllocator):
+        def borrow(self, length):
+            raise self.exc
+
+    alloc = Failing()
+    enc = pa.KernelCommandEncoder(lib, stream, scratch=alloc)
+    token, _ = _attention(pa, 8, 4, 1, 1000, 256, "bf16")  # needs its partials
+    for call in ("small_grid", "few_rows", "runs"):
+        kern, _ = CALLS[call](pa)
+        for exc in (MemoryError(), pa.PopcornError(pa.PopcornError.GPU_OUT_OF_MEMORY, "none")):
+            alloc.exc = exc
+            before = enc.stats()["dispatches"]
+            enc.encode(kern)
+            assert enc.stats()["dispatches"] == before + 1
+            with pytest.raises(pa.PopcornError) as e:
+                enc.encode(token)
+            assert e.value.__cause__ is exc and e.value.code == getattr(exc, "code", pa.PopcornError.TENSOR_ALLOCATION_FAILED)
+        alloc.exc = RuntimeError("lost track of a buffer")
+        with pytest.raises(pa.PopcornError) as e:
+            enc.encode(kern)
+        assert e.value.__cause__ is alloc.exc and e.value.code == pa.PopcornError.GPU_INTERNAL
+    stream.synchronize()
