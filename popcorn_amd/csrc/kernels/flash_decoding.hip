@@ -519,8 +519,7 @@ __device__ void fd_reduce(const float *__restrict__ pO, const float *__restrict_
 
     float mr = -INFINITY, lr = 0.0f, acc = 0.0f;
     for (uint32_t k0 = kBeg; k0 < kEnd; k0 += kReduceBatch) {
-        // entries past the range repeat the last one and are masked below (its O
-        // as well as its weight: 0 times an infinity is a NaN)
+        // entries past the range repeat the last one and are masked below
         const uint32_t kl = min(k0 + (lane % kReduceBatch), kEnd - 1);
         const float mv = m[kl], lv = l[kl];
         float ok[kReduceBatch];
@@ -543,7 +542,7 @@ __device__ void fd_reduce(const float *__restrict__ pO, const float *__restrict_
         for (int i = 0; i < kReduceBatch; ++i) {
             const float e = pk::fast_exp(mk[i] - mx);
             const float b = (k0 + i < kEnd && mk[i] != -INFINITY) ? e : 0.0f;
-            acc += (k0 + i < kEnd ? ok[i] : 0.0f) * b;
+            acc += ok[i] * b;
             lr += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lv), i)) * b;
         }
         mr = mx;
