@@ -500,8 +500,41 @@ private:
         rowTiles_ = hdp <= 128 ? 4 : hdp == 256 ? 2 : 1;
         while (rowTiles_ > 1 && (R <= 8 * rowTiles_ || blocks(rowTiles_) * cdiv(steps, 8) < cus)) rowTiles_ /= 2;
         rowsP_ = steps <= 12 ? 1 : std::clamp<int64_t>(cus / blocks(rowTiles_), 1, cdiv(steps, 4));
+        if (fd_.lpk && !rowsFaster(hdp, keys, blocks(rowTiles_))) rowTiles_ = 0;
         rowsName_ = std::string("flash_attention_rows_") + tag(t) + "_" + tag(out_.dataType) + "_d" + std::to_string(hdp) +
                     "_r";
+    }
+
+    // Whether the few-row kernels, in `blocks` blocks per partition, are faster
+    // than the one-row kernels: by estimates (us) fitted to both on 1600 shapes
+    // (13 head layouts, 2-31 rows, 31-9000 keys, 1 and 4 sequences). The latter
+    // read K and V once per row, mostly from the caches (V, MB), and grow with
+    // it; the former have the longer chain of latencies, in steps per wave, and
+    // at Hd 512 twice that (their registers spill 62 of 512, and a block is the
+    // only one on its CU). The margins leave 4 of the shapes over 2% slower, the
+    // worst 5%; the few-row kernels for all of them had 540, the worst 3.2 times
+    // (8 heads on 4, us one-row and few-row: Hd 256, 2 rows x 700 keys 8.4 and
+    // 11.0, 8 x 500 8.6 and 11.4, 8 x 1500 12.8 and 11.5, 31 x 200 10.5 and 9.4;
+    // Hd 512, 2 x 300 10.4 and 29.4, 31 x 9000 271 and 70). Head dims that the
+    // one-row kernels have only their any-dim form for are always faster here
+    // (Hd 200, 6 x 500: 23 and 10; Hd 320, 6 x 500: 27 and 17).
+    bool rowsFaster(int64_t hdp, int64_t keys, int64_t blocks) const {
+        struct {
+            double one, step1, wave1;                 // one partition: base, per step, per step of a wave
+            double parts, wave, mbKeys, mbParts, margin;  // several, with a combine
+        } const fits[] = {{3.3, 0.05, 0.58, 7.1, 0.67, 0.02, 1.0, 0.95},
+                          {3.8, 0.16, 0.62, 7.5, 0.93, 0.05, 0.9, 0.95},
+                          {4.9, 0.36, 0.95, 9.2, 1.70, 0.06, 0.5, 0.85},
+                          {9.3, 1.00, 3.70, 19.4, 0.50, 0.185, 0.7, 0.75}};
+        const auto &f = fits[hdp == 64 ? 0 : hdp == 128 ? 1 : hdp == 256 ? 2 : 3];
+        const int64_t steps = cdiv(keys, 32), waveSteps = cdiv(cdiv(steps, rowsP_), 4), rows = d_.B * d_.Nq * d_.Sq;
+        const double rowMB = (double)d_.Hd * 4e-6, g = fd_.gmax;
+        const double V = (double)(d_.B * d_.Nkv * ngroups_ * d_.Sq * keys) * rowMB;
+        const double perRow = 6.3 + 0.2 * g * (double)(d_.Hd / 64) + (0.015 + 0.05 * g) * V + (double)(rows * P_) * rowMB;
+        if (rowsP_ == 1 && steps <= 12)
+            return f.one + f.step1 * (double)steps + f.wave1 * (double)waveSteps < (hdp < 512 ? 0.95 : f.margin) * perRow;
+        return f.parts + f.wave * (double)(waveSteps * rowTiles_) + f.mbKeys * (double)(blocks * keys) * rowMB +
+                   f.mbParts * (double)(rows * rowsP_) * rowMB < f.margin * perRow;
     }
 
     // Runs (pairTiles 3): calls whose tiles leave CUs idle cut every tile's
@@ -586,6 +619,7 @@ private:
         reduceName_ = std::string("flash_decoding_reduce_") + tag(out_.dataType) + "_ext";
         ngroups_ = f.ngroups;
         P_ = f.P;
+        fd_ = f;
     }
 
     Tensor q_, k_, v_, out_, pos_;
@@ -600,6 +634,7 @@ private:
     bool pairTiles_ = false;
     int64_t runLength_ = 0, runsPerHead_ = 0;  // runs of key steps (0: none)
     int64_t rowTiles_ = 0, rowsP_ = 1;         // a few rows on the matrix cores (0: not)
+    FdPlan fd_;
     std::string rowsName_;                     // up to its number of row tiles
     bool rows16_ = false;  // the 16-rows-per-wave kernel: 8 waves per 128-row tile (4 per 64 at Hd 512 and in f32)
     int64_t hdp_ = 0;      // the tiled kernel's head dim: Hd padded to 64, 128, 256 or 512

@@ -30,7 +30,7 @@ def test_rows_rule():
         return _kernel(pa, t, 1, Nq, Nkv, Sq, Sk, Sk, Hd, **kw).function_names
 
     assert name(8, 4, 8, 4104) == ["flash_attention_rows_bf16_bf16_d256_r1", "flash_decoding_reduce_bf16_ext"]
-    assert name(8, 4, 8, 384) == ["flash_attention_rows_bf16_bf16_d256_r1"]  # 12 steps: one partition
+    assert name(8, 4, 31, 200) == ["flash_attention_rows_bf16_bf16_d256_r1"]  # up to 12 steps: one partition
     assert name(32, 8, 31, 30000, 128)[0] == "flash_attention_rows_bf16_bf16_d128_r4"
     assert name(8, 8, 2, 200, 72, ot="f32") == ["flash_attention_rows_bf16_f32_d128_r1"]
     old = "flash_decoding_partial_"
@@ -43,6 +43,12 @@ def test_rows_rule():
     q = pa.Tensor(FAKE + 2, (1, 8, 8, 256), "bf16")
     assert name(8, 4, 8, 4104, q=q)[0].startswith(old)
     assert name(8, 4, 8, 4104, ot="f16")[0].startswith(old)
+    # measured both ways at Hd 256 and 512: a longer chain of key steps per wave
+    # than the one-row kernels', until these read K and V too often
+    for case, rows in {(8, 4, 2, 700): False, (8, 4, 8, 384): False, (8, 4, 8, 1500): True, (16, 16, 2, 300): False,
+                       (8, 1, 2, 300): True, (8, 4, 2, 64): True, (8, 4, 31, 300, 512): False, (8, 4, 31, 5000, 512): True,
+                       (16, 16, 2, 2000, 512): False, (16, 16, 2, 500, 128): False, (8, 2, 6, 500, 320): True}.items():
+        assert name(*case)[0].startswith("flash_attention_rows_" if rows else old), case
 
 
 @pytest.mark.gpu
@@ -52,7 +58,8 @@ def test_rows_rule():
     (1, 4, 2, 8, 33, 40, 256, (0, -1)),         # 16 rows exactly; a second step of one key
     (2, 6, 2, 11, 500, 512, 128, (0, -1)),      # 33 rows: a third tile of one row; 16 steps: partitions
     (1, 8, 1, 31, 1100, 1100, 256, (0, -1)),    # 248 rows of one KV head
-    (1, 2, 1, 5, 700, 701, 512, (0, -1)),
+    (1, 16, 2, 24, 700, 701, 512, (0, -1)),
+    (1, 2, 1, 5, 700, 701, 400, (0, -1)),       # padded to 512
     (1, 4, 4, 3, 450, 450, 200, (2, -1)),       # padded head dim, every key
     (1, 4, 2, 9, 900, 1000, 72, (1, 100)),      # a window: most partitions of the keys unseen
     (1, 4, 1, 20, 600, 600, 128, (1, 3)),
@@ -100,10 +107,12 @@ def test_rows_wide_score_range(t):
     from gpu_util import EPS, download, gpu_env, rounded, upload
 
     pa, lib, stream, enc = gpu_env()
-    q, k = (rounded(3.0 * O.normal(s, sh), t) for s, sh in ((1, (1, 4, 7, 256)), (2, (1, 2, 640, 256))))
+    q, k = (rounded(3.0 * O.normal(s, sh), t) for s, sh in ((1, (1, 4, 31, 256)), (2, (1, 2, 640, 256))))
     v = rounded(O.normal(3, (1, 2, 640, 256)), t)
-    out = pa.Tensor.empty([1, 4, 7, 256], t)
-    enc.encode(_kernel(pa, t, 1, 4, 2, 7, 640, 640, 256, (0, -1), 1.0, upload(pa, q, t), upload(pa, k, t), upload(pa, v, t), out))
+    out = pa.Tensor.empty([1, 4, 31, 256], t)
+    kern = _kernel(pa, t, 1, 4, 2, 31, 640, 640, 256, (0, -1), 1.0, upload(pa, q, t), upload(pa, k, t), upload(pa, v, t), out)
+    assert kern.function_names[0].startswith("flash_attention_rows_")
+    enc.encode(kern)
     stream.synchronize()
     assert_out(download(out, stream), O.attention_naive(q, k, v, 1.0), EPS[t], t, "wide range")
 
@@ -127,7 +136,7 @@ def _own_keys(q, k, v, scale, mask=(0, -1)):
 # every kernel of the rule, by a call that takes it
 FORMS = [(1, 4, 2, 4, 300, 64, "d64_r1"), (8, 32, 8, 8, 1030, 64, "d64_r2"), (8, 32, 8, 16, 1030, 64, "d64_r4"),
          (1, 8, 4, 8, 1500, 128, "d128_r1"), (8, 32, 8, 8, 1030, 128, "d128_r2"), (8, 32, 8, 16, 1030, 128, "d128_r4"),
-         (1, 8, 4, 8, 1500, 256, "d256_r1"), (8, 16, 8, 16, 1030, 256, "d256_r2"), (1, 8, 2, 8, 1500, 512, "d512_r1")]
+         (1, 8, 4, 8, 1500, 256, "d256_r1"), (8, 16, 8, 16, 1030, 256, "d256_r2"), (1, 8, 2, 24, 1500, 512, "d512_r1")]
 
 
 @pytest.mark.gpu
@@ -169,14 +178,14 @@ def test_rows_non_finite_values(t, B, Nq, Nkv, Sq, Sk, Hd, form):
     pa, lib, stream, enc = gpu_env()
     q = rounded(O.normal(Sq, (B, Nq, Sq, Hd)), t)
     k, v = (rounded(O.normal(Sk + i, (B, Nkv, Sk, Hd)), t) for i in (1, 2))
-    first = Sk - Sq  # the first query's own key
-    for mask in ((0, -1), (1, 70)):
+    first, win = Sk - Sq, 1000 if Hd == 512 else 70  # the first query's own key; a window that takes these kernels
+    for mask in ((0, -1), (1, win)):
         kk, vv = k.copy(), v.copy()
         kk[:, :, Sk - 1], vv[:, :, Sk - 2] = np.nan, np.nan
         if mask[0] == 0:
             vv[:, :, 40, Hd - 3] = np.inf
         else:
-            vv[:, :, first - 70], kk[:, :, first - 71], vv[:, :, first - 75] = -np.inf, np.nan, np.nan
+            vv[:, :, first - win], kk[:, :, first - win - 1], vv[:, :, first - win - 5] = -np.inf, np.nan, np.nan
             vv[:, :, first - 5, 1] = -np.inf  # inside every window
         out = upload(pa, np.zeros(q.shape, np.float32), t)
         kern = _kernel(pa, t, B, Nq, Nkv, Sq, Sk, Sk, Hd, mask, None, upload(pa, q, t), upload(pa, kk, t), upload(pa, vv, t), out)
