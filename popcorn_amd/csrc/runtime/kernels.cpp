@@ -1689,9 +1689,14 @@ std::unique_ptr<Kernel> RMSNorm(const Tensor &x, const Tensor *weight, const Ten
     // or 64 lanes per row (rmsnorm_lanes; 8 rows of 2304, bf16: 3.5 us against
     // 3.9 on a block per row; fewer rows keep that). Blocks of one wave for
     // 64-lane rows and where four would leave CUs idle (1000 x 2304: 4.4
-    // against 4.6 us; 8000 x 256: 3.5 against 3.25).
+    // against 4.6 us; 8000 x 256: 3.5 against 3.25). Long f32 rows, whose block
+    // loads a vector per lane, keep a block per row while there are no more of
+    // them than the CUs hold (f32, us block per row and lanes: 8 x 1536 equal, 8
+    // x 2304 3.2 and 4.0, 200 x 2304 3.5 and 4.2, 256 x 2304 4.8 and 4.3; 200 x
+    // 4096 4.4 and 5.6, 300 x 4096 6.1 and 6.3, 600 x 4096 7.9 and 7.2).
     const int64_t perVec = 16 / stride(x.dataType), nvec = cdiv(hiddenSize, perVec);
-    if (rowCount >= 8 && hiddenSize % perVec == 0 && nvec <= 1024 && aligned16(x.data) && aligned16(out.data) &&
+    const bool longF32 = x.dataType == DataType::f32 && nvec >= 384 && rowCount < (nvec > 768 ? 2 : 1) * (int64_t)deviceCUs();
+    if (rowCount >= 8 && hiddenSize % perVec == 0 && nvec <= 1024 && !longF32 && aligned16(x.data) && aligned16(out.data) &&
         (!weight || aligned16(weight->data)) && rowCount <= UINT32_MAX) {
         const int64_t lanes = nvec <= 16 ? 16 : nvec <= 32 ? 32 : 64;
         const int vectors = nvec <= 64 ? 1 : nvec <= 256 ? 4 : nvec <= 512 ? 8 : 16;

@@ -19,7 +19,10 @@ def test_rows_rule():
                                   pa.Tensor(FAKE, [rows, H], t), eps=1e-6).describe()
 
     assert name(8, 2304) == "rmsnorm_rows_bf16_l64_v8" and name(8000, 256) == "rmsnorm_rows_bf16_l32_v1"
-    assert name(100, 128, "f16") == "rmsnorm_rows_f16_l16_v1" and name(9, 4096, "f32") == "rmsnorm_rows_f32_l64_v16"
+    assert name(100, 128, "f16") == "rmsnorm_rows_f16_l16_v1" and name(600, 4096, "f32") == "rmsnorm_rows_f32_l64_v16"
+    # long f32 rows: a block per row while they are few
+    assert name(9, 4096, "f32") == "rmsnorm" and name(400, 4096, "f32") == "rmsnorm" and name(255, 1536, "f32") == "rmsnorm"
+    assert name(256, 1536, "f32") == "rmsnorm_rows_f32_l64_v8" and name(9, 1528, "f32") == "rmsnorm_rows_f32_l64_v8"
     assert name(7, 2304) == "rmsnorm_bf16" and name(100, 2300) == "rmsnorm_bf16" and name(100, 8200) == "rmsnorm_bf16"
     assert name(100, 256, x_ptr=FAKE + 2) == "rmsnorm_bf16" and name(100, 256, w_ptr=FAKE + 4) == "rmsnorm_bf16"
 
@@ -35,6 +38,8 @@ def test_rows_vs_oracle(t, rows, H, weight, add_one):
     from gpu_util import EPS, download, gpu_env, rounded, upload
 
     pa, lib, stream, enc = gpu_env()
+    if t == "f32" and H >= 1536:
+        rows += 512  # fewer long f32 rows take a block each
     x = rounded(O.normal(rows + H, (rows, H)), t)
     x[rows // 2] = 0.0  # a row of zeros: its scale is 1 / sqrt(eps)
     w = O.normal(H, (H,), mean=1.0, std=0.1) if weight else None
