@@ -542,11 +542,14 @@ private:
     // merge kernel. L is the one of least estimated time,
     //   rounds x L x t + 9 us + 8 us + 0.2 us per MB of partials,
     // and runs are taken where that is under 0.9 of the whole or paired
-    // tiles' time, longest block x t + 9 us (+ 10 us for pairs' exchange),
-    // with t the time of a step (us, one block per CU; MI355X, fitted to L
-    // swept over 9 shapes per dtype). bf16, Hd 256, us before -> after: 500
-    // rows x 8692 keys, 8 heads 377 -> 68; 48 x 16000 684 -> 42; 1000 x 1000
-    // 43 -> 33; Hd 128, 300 x 3000, 32 heads 96 -> 46. Calls of under 768
+    // tiles' time, longest block x t + 9 us (for pairs, which exchange their
+    // halves, + 10 us at Hd 256 and + 4 at 64 and 128: with 10 there too, short
+    // prompts took runs and got slower, 768 rows, 24 heads, Hd 64, f16 19.3 ->
+    // 24.0 us), with t the time of a step (us, one block per CU; MI355X, fitted
+    // to L swept over 9 shapes per dtype; over 300 more, of 768 to 16000 keys,
+    // none that takes runs is over 1% slower for it). bf16, Hd 256, us before ->
+    // after: 500 rows x 8692 keys, 8 heads 377 -> 68; 48 x 16000 684 -> 42; 1000
+    // x 1000 43 -> 33; Hd 128, 300 x 3000, 32 heads 96 -> 46. Calls of under 768
     // keys stay in one launch (a 640-key call's blocks run at most 12 steps
     // as pairs).
     void planRuns() {
@@ -561,7 +564,7 @@ private:
         if (pairTiles_) {
             double longest = 0.0;
             for (int64_t i = 0; i < nQT / 2; ++i) longest = std::max(longest, 0.5 * (double)(n[i] + n[nQT - 1 - i]) + 1.0);
-            best = longest * t + 19.0;
+            best = longest * t + (hdp_ == 256 ? 19.0 : 13.0);
         }
         best *= 0.9;
         for (int64_t L = 1; L < most; ++L) {

@@ -32,6 +32,7 @@ def test_runs_rule():
     assert runs(8, 500, 8692) and runs(8, 1000, 1000) and runs(32, 300, 3000, 128) and runs(8, 100, 5000, 64)
     assert runs(8, 200, 2500, mask=(2, -1))
     assert not runs(2, 640, 640)              # under 768 keys: one launch
+    assert not runs(24, 768, 768, 64) and not runs(16, 900, 900, 128)  # pairs are faster
     assert not runs(16, 2048, 2048)           # a tile per CU
     assert not runs(8, 500, 8692, 512) and not runs(8, 500, 8692, t="f32")  # whole tiles only
     assert not runs(16, 1000, 4000, mask=(1, 64))  # a window of 7 steps: nothing to cut
