@@ -977,6 +977,7 @@ const SmallTile kSmallTiles[] = {{{64, 64, 256, "f64x64"}, 2, 0.313, 0.500, 0.2}
                                  {{128, 128, 256, "e128x128"}, 2, 0.790, 1.209, 0.6},
                                  {{128, 128, 256, "f128x128"}, 1, 0.604, 0.662, 1.6},
                                  {{256, 256, 512, "e256x256"}, 1, 1.620, 1.932, 0.4}};
+constexpr int kE128 = 2;
 
 bool gemmSmallGrid(int64_t m, int64_t n, int64_t k) {
     return (double)m * (double)n * (double)k >= 0x1p29 && cdiv(m, 128) * cdiv(n, 128) <= 2 * (int64_t)deviceCUs() &&
@@ -991,7 +992,7 @@ struct GemmPlan {
 GemmPlan gemmSmallPlan(int64_t m, int64_t n, int64_t k, bool maySplit) {
     const int64_t cus = deviceCUs(), stages = cdiv(k, 64);
     GemmPlan best{kSmallTiles[0].tile, 1};
-    double bestUs = 1e30;
+    double bestUs = 1e30, unsplit128 = 0.0;
     for (const SmallTile &t : kSmallTiles) {
         const int64_t tiles = cdiv(m, t.tile.bm) * cdiv(n, t.tile.bn);
         // a split takes at least 4 stages; more than 16 were never the fastest
@@ -1001,12 +1002,22 @@ GemmPlan gemmSmallPlan(int64_t m, int64_t n, int64_t k, bool maySplit) {
             double us = (double)rounds * (per * t.full + t.block);
             if (rest) us += per * (t.alone + (t.full - t.alone) * over) + t.block;
             if (s > 1) us += 4.3 + 0.14 * 8e-6 * (double)s * (double)m * (double)n;
+            if (s == 1 && &t == &kSmallTiles[kE128]) unsplit128 = us;
             if (us < bestUs) {
                 bestUs = us;
                 best = GemmPlan{t.tile, s};
             }
         }
     }
+    // 128 x 128 tiles of whole stages on more than one but not two full rounds
+    // of the CUs run up to 30% faster than their estimate (which is near on fewer
+    // tiles), so splits of 256 x 256 must beat it by more there: M 389, K 4096, N
+    // 14336, bf16: 50.9 us, split 60.4; M 1156, K 4096, N 4096 46.4 and 52.5; but
+    // M 1015, K 14336, N 4096 152 and 115 (300 shapes: with 0.85 none is over 4%
+    // slower than unsplit, 3 give up 3 to 17%).
+    const int64_t tiles = cdiv(m, 128) * cdiv(n, 128);
+    if (best.splits > 1 && best.tile.bm == 256 && k % 64 == 0 && tiles > cus && bestUs > 0.85 * unsplit128)
+        best = GemmPlan{kSmallTiles[kE128].tile, 1};
     return best;
 }
 

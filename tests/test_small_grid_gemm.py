@@ -26,6 +26,9 @@ def test_small_grid_plan():
     # few 128 x 128 tiles: a smaller tile, or K split over blocks
     assert _names(137, 9216, 2304)[1] == "matmul_splitk_reduce_bf16"
     assert _names(1000, 2304, 1024) == ["matmul_mfma_bf16_bf16_bf16_f64x64"]
+    # between one and two 128 x 128 tiles per CU: split only for a clear gain
+    assert _names(389, 4096, 14336) == ["matmul_mfma_bf16_bf16_bf16_e128x128"] and len(_names(1156, 4096, 4096)) == 1
+    assert len(_names(1153, 24576, 3072)) == 2 and len(_names(403, 4896, 10227)) == 2
     # C off 16-byte alignment: the reduction's vector stores are out, one pass
     assert len(_names(137, 9216, 2304, out_ptr=FAKE + 2)) == 1
     # under 2^29 multiply-adds: one 128 x 128 pass
