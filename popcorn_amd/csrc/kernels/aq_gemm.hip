@@ -22,12 +22,16 @@
 // free).
 //
 // aq_gemm: a block of 4 waves takes a 128 x 128 tile of C, each wave 128 x 32
-// (4 x 1 MFMA tiles), so each packed word is unpacked by one wave only: the
-// vector ALU work (unpacking, the FMAs of s * D) adds to the products' time.
-// Waves of 64 x 64 read fewer fragments but unpack every word twice: 9
-// products back to back, each, M 1000, K 9216, N 2304: 137 -> 124 us; M 2048,
-// K 2304, N 9216: 147 -> 137; M 777: 66 -> 61 (with pauses between them, where
-// the clock is higher: 59.7 -> 59.3, and M 71: 27.0 -> 25.9). Per group the
+// (4 x 1 MFMA tiles) or 64 x 64 (2 x 2). In the first form each packed word is
+// unpacked by one wave only, and the vector ALU work (unpacking, the FMAs of s *
+// D) adds to the products' time; the second unpacks every word twice but reads
+// half the X' fragments from LDS, 32 KB a group and block. The first starts
+// sooner (K 2048, N 2304, M 2048, 32 groups a block: 51.1 -> 48.0 us) and wins
+// with more than two blocks per CU, where the blocks' LDS reads and ALU work
+// interleave (K 3072, N 24576, M 512: 133 -> 120; M 300: 116 -> 109); with one
+// round of blocks and many groups in each the second does (K 9216, N 2304, M
+// 2048: 202 -> 193, M 3000 228 -> 211; K 4096, N 4096, M 2048: 111 -> 107). Per
+// group the
 // block copies the X' tile (128 x 64 bf16), the packed words, the columns'
 // scale and bias words and the rows'
 // X_g into LDS, three groups in flight (below). Rows past M and columns
@@ -108,7 +112,8 @@ __device__ inline void wait_vm() {
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-template <typename O, bool SPLIT>
+// WN waves across the tile's columns: 4 (each 128 x 32) or 2 (64 x 64).
+template <typename O, bool SPLIT, int WN>
 __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restrict__ S, const uint16_t *__restrict__ Bi,
                         const uint16_t *__restrict__ Xp, const float *__restrict__ Xs, typename O::storage *__restrict__ C,
                         float *__restrict__ P, const AffineQMatmulConstants &p) {
@@ -119,8 +124,8 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
     const uint32_t pm = blockIdx.x % nM, pn = blockIdx.x / nM;  // blocks sharing weights run together
     const uint32_t bm = pm * BM, bn = pn * BN;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    constexpr int MI = BM / 32, NI = 1;  // the wave's tiles of 32 x 32
-    const uint32_t wn = wave * 32;
+    constexpr int MI = BM / 32 * WN / 4, NI = BN / 32 / WN;  // the wave's tiles of 32 x 32
+    const uint32_t wm = wave / WN * (MI * 32), wn = wave % WN * (NI * 32);
     const uint32_t r = lane & 31, h = lane >> 5;
 
     // buffer resources over whole operands (the host keeps each under 2^31 bytes)
@@ -193,7 +198,7 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
             u32x4 a[MI], b[NI];
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi) {
-                const uint32_t row = mi * 32 + r, c = 4 * h + kk;
+                const uint32_t row = wm + mi * 32 + r, c = 4 * h + kk;
                 a[mi] = *reinterpret_cast<const u32x4 *>(sX + row * 128 + ((c ^ ((row >> 1) & 7)) << 4));
             }
 #pragma unroll
@@ -219,7 +224,7 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
             cb[ni] = bias - 128.0f * cs[ni];
         }
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi) cx[mi] = sG[mi * 32 + r];
+        for (int mi = 0; mi < MI; ++mi) cx[mi] = sG[wm + mi * 32 + r];
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
@@ -281,7 +286,7 @@ __device__ void aq_gemm(const uint32_t *__restrict__ Wp, const uint16_t *__restr
             if (col >= N) continue;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const uint32_t m = bm + mi * 32 + (i / 4) * 8 + h * 4 + (i % 4);
+                const uint32_t m = bm + wm + mi * 32 + (i / 4) * 8 + h * 4 + (i % 4);
                 if (m >= M) continue;
                 if constexpr (SPLIT) {
                     P[((uint64_t)blockIdx.y * M + m) * N + col] = acc[mi][ni][i];
@@ -299,22 +304,26 @@ POPCORN_KERNEL void __launch_bounds__(256)
     aq_gemm_prep(x, xp, xs, p);
 }
 
-#define AQ_GEMM(name, O)                                                                                  \
+#define AQ_GEMM(name, O, WN)                                                                              \
     POPCORN_KERNEL void __launch_bounds__(256)                                                            \
         name(const uint32_t *w, const uint16_t *s, const uint16_t *b, const uint16_t *xp, const float *xs, \
              O::storage *c, AffineQMatmulConstants p) {                                                   \
-        aq_gemm<O, false>(w, s, b, xp, xs, c, nullptr, p);                                                \
+        aq_gemm<O, false, WN>(w, s, b, xp, xs, c, nullptr, p);                                            \
     }
-
 // f32 partial tiles of a K split (gridDim.y splits), for matmul_splitk_reduce_*
-POPCORN_KERNEL void __launch_bounds__(256)
-    aq_gemm_mfma_bf16_bf16_splitk_b4_g64(const uint32_t *w, const uint16_t *s, const uint16_t *b, const uint16_t *xp,
-                                         const float *xs, float *partial, AffineQMatmulConstants p) {
-    aq_gemm<pk::F32, true>(w, s, b, xp, xs, nullptr, partial, p);
-}
+#define AQ_GEMM_SPLIT(name, WN)                                                                           \
+    POPCORN_KERNEL void __launch_bounds__(256)                                                            \
+        name(const uint32_t *w, const uint16_t *s, const uint16_t *b, const uint16_t *xp, const float *xs, \
+             float *partial, AffineQMatmulConstants p) {                                                  \
+        aq_gemm<pk::F32, true, WN>(w, s, b, xp, xs, nullptr, partial, p);                                 \
+    }
 
 using pk::BF16;
 using pk::F32;
 
-AQ_GEMM(aq_gemm_mfma_bf16_bf16_bf16_b4_g64, BF16)
-AQ_GEMM(aq_gemm_mfma_bf16_bf16_f32_b4_g64, F32)
+AQ_GEMM_SPLIT(aq_gemm_mfma_bf16_bf16_splitk_b4_g64, 4)
+AQ_GEMM_SPLIT(aq_gemm_mfma_bf16_bf16_splitk_b4_g64_w64, 2)
+AQ_GEMM(aq_gemm_mfma_bf16_bf16_bf16_b4_g64, BF16, 4)
+AQ_GEMM(aq_gemm_mfma_bf16_bf16_bf16_b4_g64_w64, BF16, 2)
+AQ_GEMM(aq_gemm_mfma_bf16_bf16_f32_b4_g64, F32, 4)
+AQ_GEMM(aq_gemm_mfma_bf16_bf16_f32_b4_g64_w64, F32, 2)

@@ -2142,8 +2142,7 @@ public:
         return t;
     }
     std::string describe() const override {
-        return splits() > 1 ? std::string("aq_gemm_prep_bf16,aq_gemm_mfma_bf16_bf16_splitk_b4_g64,") + reduceName()
-                            : std::string("aq_gemm_prep_bf16,") + mainName();
+        return "aq_gemm_prep_bf16," + mainName() + (splits() > 1 ? "," + reduceName() : std::string());
     }
     void encode(KernelCommandEncoder &enc) const override {
         const int64_t m = qc_.M, k = qc_.K, g = qc_.kGroups, n = qc_.N, tiles = cdiv(m, 128) * cdiv(n, 128);
@@ -2166,7 +2165,7 @@ public:
                     DispatchSize ds;
                     ds.grid = dim3((unsigned)tiles, (unsigned)s, 1);
                     ds.block = dim3(kBlock, 1, 1);
-                    FixedDispatch gemm("aq_gemm_mfma_bf16_bf16_splitk_b4_g64",
+                    FixedDispatch gemm(mainName(),
                                        {{b_.packedValues, kRead}, {b_.scales, kRead}, {bias, kRead}, {xp, kRead},
                                         {xs, kRead}, {part, kWrite}},
                                        {bytesOf(qc_)}, ds);
@@ -2193,7 +2192,16 @@ private:
         const bool reducible = ((int64_t)qc_.M * qc_.N) % 4 == 0 && aligned16(c_.data);
         return reducible && s >= 2 ? s : 1;
     }
-    std::string mainName() const { return std::string("aq_gemm_mfma_bf16_bf16_") + tag(c_.dataType) + "_b4_g64"; }
+    // Waves of 64 x 64 where all blocks run in one round of two per CU with more
+    // than 36 groups each, else of 128 x 32 (aq_gemm.hip). Over 260 shapes, 128 x
+    // 32 against 64 x 64: up to 36 groups 2.3% faster (2 of 97 over 2% slower, the
+    // worst 4%), more blocks 5% faster (none over 2% slower), the rest equal on
+    // average with 45 of 127 over 2% slower, the worst 10%.
+    std::string mainName() const {
+        const int64_t s = splits(), blocks = cdiv((int64_t)qc_.M, 128) * cdiv((int64_t)qc_.N, 128) * s;
+        const bool w64 = blocks <= 2 * (int64_t)deviceCUs() && cdiv((int64_t)qc_.kGroups, s) > 36;
+        return std::string("aq_gemm_mfma_bf16_bf16_") + (s > 1 ? "splitk" : tag(c_.dataType)) + "_b4_g64" + (w64 ? "_w64" : "");
+    }
     std::string reduceName() const { return std::string("matmul_splitk_reduce_") + tag(c_.dataType); }
     Tensor a_;
     AffineQuantizedTensor b_;

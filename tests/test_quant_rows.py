@@ -97,3 +97,39 @@ def test_rows_vs_oracle(M, N, K, bias):
     packed, s, b, _ = quantize_q4(0.05 * rng.standard_normal((N, K)).astype(np.float32), bias=bias)
     x = rounded(rng.standard_normal((M, K)).astype(np.float32), "bf16")
     assert_out(_run(x, packed, s, b, N, K), O.aq_matmul(x, packed, s, b, N, K), EPS["bf16"], "bf16", f"{M}x{N}x{K} bias={bias}")
+
+
+def test_prompt_wave_forms_rule():
+    # waves of 64 x 64 in one round of blocks with more than 36 groups each
+    name = "aq_gemm_mfma_bf16_bf16_"
+    assert _names(129, 1031, 2432)[1] == name + "bf16_b4_g64_w64" and _names(129, 1031, 2304)[1] == name + "bf16_b4_g64"
+    assert _names(1100, 2900, 4864)[1] == name + "splitk_b4_g64_w64" and _names(1100, 2900, 4608)[1] == name + "splitk_b4_g64"
+    assert _names(777, 9216, 3072)[1] == name + "bf16_b4_g64_w64"   # 504 blocks
+    assert _names(1000, 9216, 3072)[1] == name + "bf16_b4_g64"      # 576
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(129, 1031, 2432), (1100, 2900, 4864)])  # whole K, and split
+def test_prompt_wave_form_integer_exact(M, N, K):
+    # small integers: every product and sum is an exact f32 integer in any order
+    from gpu_util import download, gpu_env, upload
+    from q4util import pack_q4
+
+    pa, lib, stream, enc = gpu_env()
+    rng = np.random.default_rng(M + N + K)
+    q = rng.integers(0, 16, (N, K)).astype(np.uint32)
+    s = 2.0 ** rng.integers(0, 2, (N, K // 64)).astype(np.float32)
+    b = rng.integers(-8, 8, (N, K // 64)).astype(np.float32)
+    x = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    w = pa.AffineQuantizedTensor(pa.Tensor.from_numpy(pack_q4(q).view(np.uint32), "u32"), upload(pa, s, "bf16"),
+                                 upload(pa, b, "bf16"), [N, K])
+    guard = 64
+    buf = upload(pa, np.full(M * N + guard, np.nan, np.float32), "f32")
+    k = pa.Kernels.Matmul(upload(pa, x, "bf16"), w, buf.view([M, N]))
+    assert k.function_names[1].endswith("_w64")
+    enc.encode(k)
+    stream.synchronize()
+    out = download(buf, stream)
+    assert np.isnan(out[M * N:]).all(), "wrote past C"
+    dense = q.astype(np.float64) * np.repeat(s, 64, 1) + np.repeat(b, 64, 1)
+    np.testing.assert_array_equal(out[:M * N].reshape(M, N), (x.astype(np.float64) @ dense.T).astype(np.float32))
