@@ -52,21 +52,24 @@ def test_rows_rule():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("t,ot", [("f16", "f16"), ("bf16", "bf16"), ("bf16", "f32")])
-@pytest.mark.parametrize("B,Nq,Nkv,Sq,Sk,cap,Hd,mask", [
-    (1, 2, 2, 2, 2, 2, 64, (0, -1)),            # fewer keys than a step, rows of one head
-    (1, 4, 2, 8, 33, 40, 256, (0, -1)),         # 16 rows exactly; a second step of one key
-    (2, 6, 2, 11, 500, 512, 128, (0, -1)),      # 33 rows: a third tile of one row; 16 steps: partitions
-    (1, 8, 1, 31, 1100, 1100, 256, (0, -1)),    # 248 rows of one KV head
-    (1, 16, 2, 24, 700, 701, 512, (0, -1)),
-    (1, 2, 1, 5, 700, 701, 400, (0, -1)),       # padded to 512
-    (1, 4, 4, 3, 450, 450, 200, (2, -1)),       # padded head dim, every key
-    (1, 4, 2, 9, 900, 1000, 72, (1, 100)),      # a window: most partitions of the keys unseen
-    (1, 4, 1, 20, 600, 600, 128, (1, 3)),
-    (8, 32, 8, 16, 2050, 2050, 64, (0, -1)),    # 4 row tiles per block
-    (8, 16, 8, 16, 1100, 1100, 256, (0, -1)),   # 2 row tiles per block
+@pytest.mark.parametrize("t,ot", [("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("B,Nq,Nkv,Sq,Sk,cap,Hd,mask,form", [
+    (1, 2, 2, 2, 2, 2, 64, (0, -1), "d64_r1"),             # fewer keys than a step, rows of one head
+    (1, 4, 2, 8, 33, 40, 256, (0, -1), "d256_r1"),         # 16 rows exactly; a second step of one key
+    (2, 6, 2, 11, 500, 512, 128, (0, -1), "d128_r1"),      # 33 rows: a third tile of one row; 16 steps: partitions
+    (1, 8, 1, 31, 1100, 1100, 256, (0, -1), "d256_r1"),    # 248 rows of one KV head
+    (1, 16, 2, 24, 700, 701, 512, (0, -1), "d512_r1"),
+    (1, 2, 1, 5, 700, 701, 400, (0, -1), "d512_r1"),       # padded to 512
+    (1, 4, 4, 3, 450, 450, 200, (2, -1), "d256_r1"),       # padded head dim, every key
+    (1, 4, 2, 9, 900, 1000, 72, (1, 100), "d128_r1"),      # a window: most partitions of the keys unseen
+    (1, 4, 1, 20, 600, 600, 128, (1, 3), "d128_r1"),
+    (8, 32, 8, 8, 1030, 1031, 64, (0, -1), "d64_r2"),      # 2 and 4 row tiles per block
+    (8, 32, 8, 16, 2050, 2050, 64, (0, -1), "d64_r4"),
+    (8, 32, 8, 8, 1030, 1030, 128, (0, -1), "d128_r2"),
+    (8, 32, 8, 16, 1030, 1030, 128, (0, -1), "d128_r4"),
+    (8, 16, 8, 16, 1100, 1100, 256, (0, -1), "d256_r2"),
 ])
-def test_rows_vs_oracle(t, ot, B, Nq, Nkv, Sq, Sk, cap, Hd, mask):
+def test_rows_vs_oracle(t, ot, B, Nq, Nkv, Sq, Sk, cap, Hd, mask, form):
     import oracle as O
     from conftest import assert_out
     from gpu_util import EPS, download, gpu_env, rounded, upload
@@ -79,7 +82,7 @@ def test_rows_vs_oracle(t, ot, B, Nq, Nkv, Sq, Sk, cap, Hd, mask):
     buf = upload(pa, np.full(q.size + guard, 7.0, np.float32), ot)
     kern = _kernel(pa, t, B, Nq, Nkv, Sq, Sk, cap, Hd, mask, None, upload(pa, q, t), upload(pa, k, t), upload(pa, v, t),
                    buf.view([B, Nq, Sq, Hd]))
-    assert kern.function_names[0].startswith("flash_attention_rows_")
+    assert kern.function_names[0] == f"flash_attention_rows_{t}_{ot}_{form}"
     ref = O.attention_naive(q, k, v, Hd ** -0.5, key_len=Sk, mask_kind=mask[0], window=mask[1])
 
     class Empty(pa.KernelScratchAllocator):

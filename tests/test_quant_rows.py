@@ -38,13 +38,19 @@ def test_rows_rule():
     assert _names(32, 2304, 9216)[0] == "aq_gemm_prep_bf16"
 
 
-def _run(x, packed, s, b, N, K):
-    from gpu_util import download, gpu_env, upload
+def _matrix(env, packed, s, b, N, K):
+    from gpu_util import upload
 
-    pa, lib, stream, enc = gpu_env()
+    pa = env[0]
+    return pa.AffineQuantizedTensor(pa.Tensor.from_numpy(packed.view(np.uint32), "u32"), upload(pa, s, "bf16"),
+                                    upload(pa, b, "bf16") if b is not None else None, [N, K])
+
+
+def _run(env, x, w, N):
+    from gpu_util import download, upload
+
+    pa, lib, stream, enc = env
     M, guard = x.shape[0], 64
-    w = pa.AffineQuantizedTensor(pa.Tensor.from_numpy(packed.view(np.uint32), "u32"), upload(pa, s, "bf16"),
-                                 upload(pa, b, "bf16") if b is not None else None, [N, K])
     buf = upload(pa, np.full(M * N + guard, np.nan, np.float32), "bf16")
     k = pa.Kernels.Matmul(upload(pa, x, "bf16"), w, buf.view([M, N]))
     assert k.function_names[0].startswith(PREFIX)
@@ -53,6 +59,13 @@ def _run(x, packed, s, b, N, K):
     out = download(buf, stream)
     assert np.isnan(out[M * N:]).all(), "wrote past C"
     return out[:M * N].reshape(M, N)
+
+
+@pytest.fixture(scope="module")
+def env():
+    from gpu_util import gpu_env
+
+    return gpu_env()
 
 
 SHAPES = [(3, 9216, 1024),     # two units, two waves per tile
@@ -66,28 +79,36 @@ SHAPES = [(3, 9216, 1024),     # two units, two waves per tile
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", SHAPES)
-def test_rows_integer_exact(M, N, K):
-    # x in {-1, 0, 1}, scales 1, integer biases, one nonzero x per row and
-    # chunk: sums below 2^8 are exact in f32 and in bf16, so every nibble, x,
-    # scale, bias and output index is pinned
+def test_rows_integer_exact(env, M, N, K):
+    # One x of 1 or -1 in each group of a row, at a value that the rows and the
+    # passes walk through, so that every value of K meets every row of W. The
+    # scales differ by powers of two and the biases are whole: every sum is a
+    # whole number under 2^24, exact in f32 whatever the order, and the output is
+    # its one rounding to bf16. A wrong nibble, x, scale, bias or index moves
+    # whole rows or columns by whole units.
+    import oracle as O
     from q4util import pack_q4
 
     rng = np.random.default_rng(M + N + K)
     q = rng.integers(0, 16, (N, K)).astype(np.uint32)
+    s = 2.0 ** rng.integers(0, 4, (N, K // 64)).astype(np.float32)
     b = rng.integers(-8, 8, (N, K // 64)).astype(np.float32)
-    x = np.zeros((M, K), np.float32)
-    for r in range(M):
-        x[r, rng.integers(0, K, 6)] = rng.choice([-1.0, 1.0], 6)
-    got = _run(x, pack_q4(q), np.ones((N, K // 64), np.float32), b, N, K)
-    want = x.astype(np.float64) @ (q + np.repeat(b, 64, 1)).astype(np.float64).T
-    assert np.abs(want).max() <= 256
-    np.testing.assert_array_equal(got, want.astype(np.float32))
+    dense = (q * np.repeat(s, 64, 1) + np.repeat(b, 64, 1)).astype(np.float32)
+    w, seen = _matrix(env, pack_q4(q), s, b, N, K), np.zeros(K, bool)
+    for p in range(0, 64, M):
+        x = np.zeros((M, K // 64, 64), np.float32)
+        for r in range(M):
+            x[r, :, (p + r) % 64] = rng.choice([-1.0, 1.0], K // 64)
+        x = x.reshape(M, K)
+        seen |= (x != 0).any(0)
+        np.testing.assert_array_equal(_run(env, x, w, N), O.round_to(x @ dense.T, O.BF16))
+    assert seen.all()
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("bias", [True, False])
-def test_rows_vs_oracle(M, N, K, bias):
+def test_rows_vs_oracle(env, M, N, K, bias):
     import oracle as O
     from conftest import assert_out
     from gpu_util import EPS, rounded
@@ -96,7 +117,7 @@ def test_rows_vs_oracle(M, N, K, bias):
     rng = np.random.default_rng(M * 7 + N + K)
     packed, s, b, _ = quantize_q4(0.05 * rng.standard_normal((N, K)).astype(np.float32), bias=bias)
     x = rounded(rng.standard_normal((M, K)).astype(np.float32), "bf16")
-    assert_out(_run(x, packed, s, b, N, K), O.aq_matmul(x, packed, s, b, N, K), EPS["bf16"], "bf16", f"{M}x{N}x{K} bias={bias}")
+    assert_out(_run(env, x, _matrix(env, packed, s, b, N, K), N), O.aq_matmul(x, packed, s, b, N, K), EPS["bf16"], "bf16", f"{M}x{N}x{K} bias={bias}")
 
 
 def test_prompt_wave_forms_rule():
@@ -110,19 +131,18 @@ def test_prompt_wave_forms_rule():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(129, 1031, 2432), (1100, 2900, 4864)])  # whole K, and split
-def test_prompt_wave_form_integer_exact(M, N, K):
+def test_prompt_wave_form_integer_exact(env, M, N, K):
     # small integers: every product and sum is an exact f32 integer in any order
-    from gpu_util import download, gpu_env, upload
+    from gpu_util import download, upload
     from q4util import pack_q4
 
-    pa, lib, stream, enc = gpu_env()
+    pa, lib, stream, enc = env
     rng = np.random.default_rng(M + N + K)
     q = rng.integers(0, 16, (N, K)).astype(np.uint32)
     s = 2.0 ** rng.integers(0, 2, (N, K // 64)).astype(np.float32)
     b = rng.integers(-8, 8, (N, K // 64)).astype(np.float32)
     x = rng.integers(-3, 4, (M, K)).astype(np.float32)
-    w = pa.AffineQuantizedTensor(pa.Tensor.from_numpy(pack_q4(q).view(np.uint32), "u32"), upload(pa, s, "bf16"),
-                                 upload(pa, b, "bf16"), [N, K])
+    w = _matrix(env, pack_q4(q), s, b, N, K)
     guard = 64
     buf = upload(pa, np.full(M * N + guard, np.nan, np.float32), "f32")
     k = pa.Kernels.Matmul(upload(pa, x, "bf16"), w, buf.view([M, N]))
