@@ -456,16 +456,6 @@ public:
     }
 
 private:
-    // Causal prefill with few tiles per CU: the last query tiles see up to
-    // twice the mean number of keys and, one tile per CU, set the kernel's
-    // time. Tiles with more than half the largest tile's key steps run as
-    // two blocks over the halves of their keys, merged by a second kernel.
-    // Causal prefill with at most two tiles per CU splits tiles in two
-    // (flash_attention_tiled.hip, fa_work). With at most one tile per CU a
-    // head's query tiles are paired light with heavy (tile i with nQT - 1 - i)
-    // and each pair runs as two blocks of equal work, when every pair splits
-    // its heavy tile (x >= 1 steps in the first block); otherwise the tiles
-    // with more than half the heaviest tile's steps run as two halves.
     // Key steps of 32 that query tile qt of 128 rows visits (fa_steps).
     int64_t keySteps(int64_t qt) const {
         const int64_t first = d_.Sk - d_.Sq + qt * 128, last = d_.Sk - d_.Sq + std::min(qt * 128 + 127, d_.Sq - 1);
@@ -483,8 +473,9 @@ private:
     // tile 64); else one (31 rows x 2000 keys, 8 heads on one, Hd 256: 1 tile
     // 15.3 us, 2 tiles 18.4). Partitions: one block per CU, a step per wave at
     // least (8 rows x 4104 keys, 4 KV heads: 33 partitions 12.2 us, 17 14.1,
-    // 65 13.7); up to 12 steps one partition, which needs no combine (100
-    // keys: 4.2 against 7.6 us). Before, per row: 507, 62.4 and 22.7 us.
+    // 65 13.7); up to 12 steps one partition, which needs no combine (4 heads on
+    // 2, Hd 64, 8 rows x 300 keys: 5.5 us, 500 keys in partitions 7.9). On the
+    // one-row kernels the three calls take 507, 62.4 and 22.7 us.
     void planRows() {
         const int64_t lim = int64_t{1} << 31, G = d_.Nq / d_.Nkv, R = d_.Sq * G, cus = deviceCUs();
         const DataType t = q_.dataType;
@@ -550,8 +541,10 @@ private:
     // none that takes runs is over 1% slower for it). bf16, Hd 256, us before ->
     // after: 500 rows x 8692 keys, 8 heads 377 -> 68; 48 x 16000 684 -> 42; 1000
     // x 1000 43 -> 33; Hd 128, 300 x 3000, 32 heads 96 -> 46. Calls of under 768
-    // keys stay in one launch (a 640-key call's blocks run at most 12 steps
-    // as pairs).
+    // keys keep the one launch that the tests of the paired and the split tiles
+    // hold there, not because it is the faster: runs would take 0.33 to 1 of its
+    // time (134 shapes of 32 to 767 rows and 400 to 767 keys, 0.63 on average;
+    // 8 heads on 4, Hd 256, bf16, 32 x 640: 32.4 -> 12.7 us).
     void planRuns() {
         const int64_t nQT = cdiv(d_.Sq, 128), BH = d_.B * d_.Nq, cus = deviceCUs();
         if (d_.Sk < 768 || BH * nQT >= cus) return;
@@ -585,6 +578,16 @@ private:
         }
     }
 
+    // Causal prefill with few tiles per CU: the last query tiles see up to
+    // twice the mean number of keys and, one tile per CU, set the kernel's
+    // time. Tiles with more than half the largest tile's key steps run as
+    // two blocks over the halves of their keys, merged by a second kernel.
+    // Causal prefill with at most two tiles per CU splits tiles in two
+    // (flash_attention_tiled.hip, fa_work). With at most one tile per CU a
+    // head's query tiles are paired light with heavy (tile i with nQT - 1 - i)
+    // and each pair runs as two blocks of equal work, when every pair splits
+    // its heavy tile (x >= 1 steps in the first block); otherwise the tiles
+    // with more than half the heaviest tile's steps run as two halves.
     void planTileSplit() {
         nSplit_ = 0;
         pairTiles_ = false;
