@@ -31,14 +31,12 @@
 // interleave (K 3072, N 24576, M 512: 133 -> 120; M 300: 116 -> 109); with one
 // round of blocks and many groups in each the second does (K 9216, N 2304, M
 // 2048: 202 -> 193, M 3000 228 -> 211; K 4096, N 4096, M 2048: 111 -> 107). Per
-// group the
-// block copies the X' tile (128 x 64 bf16), the packed words, the columns'
-// scale and bias words and the rows'
-// X_g into LDS, three groups in flight (below). Rows past M and columns
-// past N read zeros and are not stored. A block walks its groups one after
-// another, so with few tiles the groups are split over gridDim.y blocks per
-// tile (SPLIT): each writes its f32 partial tile to P [gridDim.y][M][N] and
-// matmul_splitk_reduce_* sums them and rounds once.
+// group the block copies the X' tile (128 x 64 bf16), the packed words, the
+// columns' scale and bias words and the rows' X_g into LDS, three groups in
+// flight (below). Rows past M and columns past N read zeros and are not stored.
+// A block walks its groups one after another, so with few tiles the groups are
+// split over gridDim.y blocks per tile (SPLIT): each writes its f32 partial tile
+// to P [gridDim.y][M][N] and matmul_splitk_reduce_* sums them and rounds once.
 #include "mfma.hpp"
 
 namespace {
