@@ -115,7 +115,7 @@ __device__ inline void fa_rows_seen(const uint16_t *__restrict__ q, const uint16
             s = pk::group_sum<16>(s) * c2;
             if (k + u >= k1 || !seen(k + u)) continue;  // a row's lanes together
             const float mn = fmaxf(m, s);
-            if (mn == -INFINITY) continue;
+            if (mn == -INFINITY && s == -INFINITY) continue;  // (a NaN is not left out, also as the first score)
             const float alpha = __builtin_amdgcn_exp2f(m - mn), w = __builtin_amdgcn_exp2f(s - mn);
             l = l * alpha + w;
             m = mn;

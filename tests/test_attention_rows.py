@@ -204,3 +204,28 @@ def test_rows_non_finite_values(t, B, Nq, Nkv, Sq, Sk, Hd, form):
             np.testing.assert_array_equal(got == np.inf, ref == np.inf, err_msg=f"{name} {mask}")
             np.testing.assert_array_equal(got == -np.inf, ref == -np.inf, err_msg=f"{name} {mask}")
         assert_out(got[ok], ref[ok], EPS[t], t, f"{name} {mask}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", ["f16", "bf16"])
+@pytest.mark.parametrize("B,Nq,Nkv,Sq,Sk,Hd,form", FORMS)
+def test_rows_nan_in_the_first_key(t, B, Nq, Nkv, Sq, Sk, Hd, form):
+    # a row whose first score is NaN gives what the one-row kernels give for it,
+    # not the attention over its other keys
+    import oracle as O
+    from gpu_util import download, gpu_env, rounded, upload
+
+    pa, lib, stream, enc = gpu_env()
+    q = rounded(O.normal(Sq, (B, Nq, Sq, Hd)), t)
+    k, v = (rounded(O.normal(Sk + i, (B, Nkv, Sk, Hd)), t) for i in (1, 2))
+    k[:, :, 0] = np.nan
+    kt, vt = upload(pa, k, t), upload(pa, v, t)
+    out = upload(pa, np.full(q.shape, 7.0, np.float32), t)
+    kern = _kernel(pa, t, B, Nq, Nkv, Sq, Sk, Sk, Hd, (0, -1), None, upload(pa, q, t), kt, vt, out)
+    assert kern.function_names[0].endswith(form)
+    enc.encode(kern)
+    for i in (0, Sq - 1):
+        one = upload(pa, np.full((B, Nq, 1, Hd), 7.0, np.float32), t)
+        enc.encode(_kernel(pa, t, B, Nq, Nkv, 1, Sk - Sq + i + 1, Sk, Hd, (0, -1), None, upload(pa, q[:, :, i:i + 1], t), kt, vt, one))
+        stream.synchronize()
+        np.testing.assert_array_equal(download(out, stream)[:, :, i], download(one, stream)[:, :, 0], err_msg=form)
