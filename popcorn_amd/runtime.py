@@ -10,6 +10,7 @@ numpy arrays (bf16 as uint16 bit patterns).
 from __future__ import annotations
 
 import ctypes as C
+import sys
 from dataclasses import dataclass
 from typing import Iterable, Optional, Sequence
 
@@ -428,9 +429,10 @@ class ScratchPool:
 class KernelScratchAllocator:
     """Base for Python allocators: override borrow(length) -> (ptr, was_reused) and release(ptr).
 
-    A borrow that has nothing to give raises MemoryError (or the PopcornError of a
-    failed allocation): kernels that can do without the scratch then run without
-    it. Any other exception ends the encode, as the cause of its PopcornError."""
+    A borrow that has nothing to give raises MemoryError (or torch's
+    OutOfMemoryError, or the PopcornError of a failed allocation): kernels that can
+    do without the scratch then run without it. Any other exception ends the
+    encode, as the cause of its PopcornError."""
 
     error = None  # what the last failed borrow raised
 
@@ -452,7 +454,9 @@ class KernelScratchAllocator:
                 self.error = e
                 if isinstance(e, PopcornError):
                     return e.code
-                return PopcornError.TENSOR_ALLOCATION_FAILED if isinstance(e, MemoryError) else PopcornError.GPU_INTERNAL
+                torch = sys.modules.get("torch")
+                none = isinstance(e, MemoryError) or (torch is not None and isinstance(e, torch.OutOfMemoryError))
+                return PopcornError.TENSOR_ALLOCATION_FAILED if none else PopcornError.GPU_INTERNAL
 
         def _release(ctx, ptr):
             self.release(ptr)

@@ -163,6 +163,8 @@ def test_graph_without_scratch(env, call, eager):
 def test_allocator_errors(env):
     # no memory: the kernels that can do without it run; any other error of the
     # allocator reaches the caller, with what it raised
+    import torch
+
     pa, lib, stream, _ = env
 
     class Failing(pa.KernelScratchAllocator):
@@ -174,7 +176,7 @@ def test_allocator_errors(env):
     token, _ = _attention(pa, 8, 4, 1, 1000, 256, "bf16")  # needs its partials
     for call in ("small_grid", "few_rows", "runs"):
         kern, _ = CALLS[call](pa)
-        for exc in (MemoryError(), pa.PopcornError(pa.PopcornError.GPU_OUT_OF_MEMORY, "none")):
+        for exc in (MemoryError(), torch.OutOfMemoryError(), pa.PopcornError(pa.PopcornError.GPU_OUT_OF_MEMORY, "none")):
             alloc.exc = exc
             before = enc.stats()["dispatches"]
             enc.encode(kern)
